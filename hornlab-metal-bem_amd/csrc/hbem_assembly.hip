@@ -128,126 +128,102 @@ __device__ __forceinline__ GD kernel_gd_far(double dx, double dy, double dz, flo
 
 constexpr int kTestsPerWave = kTileTris / 4;
 
-// Both directions of one (t, s, image) combination over the 6 x 6 rule,
-// added to dF[i][j] (test basis i on t, trial basis j on s) and dR[i][j]
-// (test basis i on s, trial basis j on t) as -4 pi DLP / jac_s; sF[i]
-// (basis on t) and sR[i] (basis on s) get 4 pi SLP / jac_s with the
-// source's unit density.  tsc = 2 area(t) scales t's weights.
-// kPrecise: the points are vertex 0 plus an offset (o = X e1 + Y e2, from
-// exact float vertices), yp holds the trial offsets yo and xa_m the FP64
-//   B_a = (v0_s - S_m v0_t) - S_m xo_a,   d = y_b - S_m x_a = yo_b + B_a,
-// and the distance and the phase are formed in FP64 (every difference is
-// then rounded relative to |d|, and k r keeps its accuracy at large k r).
-// Both triangles are flat, so the normal projections of d = y_b - S_m x_a
-// depend on one point only:
-//   d . n_s         = (v0_s - S_m x_a) . n_s          = hF[a]
-//   d . (S_m n_t)   = (y_b - S_m v0_t) . (S_m n_t)    = hR[b]
-// (differences of nearby points first, so the rounding scales with |d|).
-template <bool kComplexK, bool kSource, bool kPrecise, typename XT>
-__device__ __forceinline__ void regular_both(const XT (&xa_m)[18], const float (&hF)[6],
-                                             const float (&hR)[6], const float (&yp)[18],
-                                             float k, float krev, double krev64, float kim, float tsc,
-                                             float (&dF)[9][2],
-                                             float (&dR)[9][2], float (&sF)[3][2],
-                                             float (&sR)[3][2]) {
+// The weights of the six-point rule times the basis values take four values:
+// w phi_j at point b is kWb[group] + (j == corner of b ? kWa[group] : 0), with
+// the points {0, 2, 3} and {1, 4, 5} as groups and corners {0, 1, 2} each.  A
+// weighted basis sum is then one shared sum and one term per point (4 FMAs per
+// complex value instead of 6).
+constexpr int kRule6Corner[6] = {0, 0, 1, 2, 1, 2};
+constexpr int kRule6Group[6] = {0, 1, 0, 0, 1, 1};
+constexpr double rule6_phi(int b, int j) {
+    return j == 0 ? 1.0 - kRule6X[b] - kRule6Y[b] : (j == 1 ? kRule6X[b] : kRule6Y[b]);
+}
+struct RuleWeights {
+    float wb[2], wa[2], wc[2];  // w phi of the other corners, difference, w phi of the point's own
+};
+
+// A value kept in a vector register.  A wave64 FP32 operation issues in two
+// cycles with vector operands and in four with a scalar one (2.3 and 4.0
+// measured with two waves per SIMD), so the uniform factors of the inner loop
+// are held in vector registers.
+__device__ __forceinline__ float in_vgpr(float x) {
+    asm("" : "+v"(x));
+    return x;
+}
+
+// Brackets of a run of transcendentals.  A transcendental takes both issue
+// ports of a SIMD for 8 cycles, and FP32 operations of two waves share a cycle
+// pair only while neither has one waiting: interleaved with the other work of
+// its wave, each costs about 20 cycles.  Six evaluations' worth issued back to
+// back at raised wave priority (the other wave waits, then both pair up) take
+// 86 cycles per evaluation instead of 136, two waves per SIMD (a loop of the
+// kernel's 26 FP32 operations, fract and 3 transcendentals per evaluation).
+__device__ __forceinline__ void trans_begin() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+}
+__device__ __forceinline__ void trans_end() {
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+__device__ __forceinline__ RuleWeights rule_weights() {
+    RuleWeights w;
+    constexpr int point[2] = {0, 1};
 #pragma unroll
-    for (int a = 0; a < 6; ++a) {
-        const XT xa = xa_m[3 * a], ya = xa_m[3 * a + 1], za = xa_m[3 * a + 2];
-        float eF[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
-        float eR[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
-        float gF[2] = {0.f, 0.f};
-        float gR[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
+    for (int g = 0; g < 2; ++g) {
+        const int b = point[g];
+        w.wb[g] = in_vgpr((float)(kRule6W[b] * rule6_phi(b, 1)));
+        w.wa[g] = in_vgpr((float)(kRule6W[b] * (rule6_phi(b, 0) - rule6_phi(b, 1))));
+        w.wc[g] = in_vgpr((float)(kRule6W[b] * rule6_phi(b, 0)));
+    }
+    return w;
+}
+
+// Basis sums of complex values; sum(j) is basis j's.  kShared: s + e[j] with
+// the shared sum above; else the three sums with their own weights (6 FMAs),
+// whose rounding stays below that of the smallest weight (FP64 geometry).
+template <bool kShared>
+struct BasisSum {
+    float s[2], e[3][2];
+    __device__ __forceinline__ void clear() {
+        s[0] = s[1] = 0.0f;
 #pragma unroll
-        for (int bq = 0; bq < 6; ++bq) {
-            float r, rinv, s, c;
-            if constexpr (kPrecise) {
-                // d = yo_b + B_a in FP64; distance and phase in FP64
-                const double dxd = (double)yp[3 * bq] + xa, dyd = (double)yp[3 * bq + 1] + ya,
-                             dzd = (double)yp[3 * bq + 2] + za;
-                const double r2d = fma(dxd, dxd, fma(dyd, dyd, dzd * dzd));
-                const float r2 = fmaxf((float)r2d, 1.0e-14f);
-                rinv = __builtin_amdgcn_rsqf(r2);
-                r = r2 * rinv;
-                const double rd = (double)r + fma(-(double)r, (double)r, r2d) * (double)(0.5f * rinv);
-                double td = rd * krev64;
-                td -= rint(td);
-                s = __builtin_amdgcn_sinf((float)td);
-                c = __builtin_amdgcn_cosf((float)td);
-            } else {
-                const float dx = yp[3 * bq] - xa;
-                const float dy = yp[3 * bq + 1] - ya;
-                const float dz = yp[3 * bq + 2] - za;
-                const float r2 = fmaxf(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), 1.0e-14f);
-                rinv = __builtin_amdgcn_rsqf(r2);
-                r = r2 * rinv;
-                // phase in revolutions, reduced to [0, 1) (exact)
-                const float t = __builtin_amdgcn_fractf(r * krev);
-                s = __builtin_amdgcn_sinf(t);
-                c = __builtin_amdgcn_cosf(t);
-            }
-            float q2 = rinv * rinv;  // 1/r^2 (times the damping)
-            float damp = 1.0f;
-            if (kComplexK) {
-                damp = __expf(-kim * r);
-                q2 *= damp;
-            }
-            const float fr = kComplexK ? rinv + kim : rinv;
-            // -4 pi dG/dn = proj/r^2 * (c fr + s k, s fr - c k) e^{-kim r}
-            const float p1 = fmaf(s, k, c * fr);
-            const float p2 = fmaf(-c, k, s * fr);
-            const float uF = hF[a] * q2;
-            const float uR = -hR[bq] * q2;
-            const float wb = (float)kRule6W[bq];
-            const float w1 = wb * (float)kRule6X[bq];
-            const float w2 = wb * (float)kRule6Y[bq];
-            const float w0 = wb - w1 - w2;
-            const float f1 = p1 * uF, f2 = p2 * uF;
-            const float r1 = p1 * uR, r2v = p2 * uR;
-            eF[0][0] = fmaf(f1, w0, eF[0][0]);
-            eF[0][1] = fmaf(f2, w0, eF[0][1]);
-            eF[1][0] = fmaf(f1, w1, eF[1][0]);
-            eF[1][1] = fmaf(f2, w1, eF[1][1]);
-            eF[2][0] = fmaf(f1, w2, eF[2][0]);
-            eF[2][1] = fmaf(f2, w2, eF[2][1]);
-            eR[0][0] = fmaf(r1, w0, eR[0][0]);
-            eR[0][1] = fmaf(r2v, w0, eR[0][1]);
-            eR[1][0] = fmaf(r1, w1, eR[1][0]);
-            eR[1][1] = fmaf(r2v, w1, eR[1][1]);
-            eR[2][0] = fmaf(r1, w2, eR[2][0]);
-            eR[2][1] = fmaf(r2v, w2, eR[2][1]);
-            if (kSource) {
-                const float g = rinv * damp;
-                const float gc = c * g, gs = s * g;
-                gF[0] = fmaf(gc, wb, gF[0]);
-                gF[1] = fmaf(gs, wb, gF[1]);
-                gR[0][0] = fmaf(gc, w0, gR[0][0]);
-                gR[0][1] = fmaf(gs, w0, gR[0][1]);
-                gR[1][0] = fmaf(gc, w1, gR[1][0]);
-                gR[1][1] = fmaf(gs, w1, gR[1][1]);
-                gR[2][0] = fmaf(gc, w2, gR[2][0]);
-                gR[2][1] = fmaf(gs, w2, gR[2][1]);
-            }
-        }
-        const float wa = (float)kRule6W[a] * tsc;
-        const float ta[3] = {wa * (float)(1.0 - kRule6X[a] - kRule6Y[a]), wa * (float)kRule6X[a],
-                             wa * (float)kRule6Y[a]};
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
+        for (int j = 0; j < 3; ++j) e[j][0] = e[j][1] = 0.0f;
+    }
+    __device__ __forceinline__ void add(const RuleWeights &w, int b, float re, float im) {
+        const int g = kRule6Group[b], corner = kRule6Corner[b];
+        if constexpr (kShared) {
+            s[0] = fmaf(re, w.wb[g], s[0]);
+            s[1] = fmaf(im, w.wb[g], s[1]);
+            e[corner][0] = fmaf(re, w.wa[g], e[corner][0]);
+            e[corner][1] = fmaf(im, w.wa[g], e[corner][1]);
+        } else {
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
-                dF[3 * i + j][0] = fmaf(ta[i], eF[j][0], dF[3 * i + j][0]);
-                dF[3 * i + j][1] = fmaf(ta[i], eF[j][1], dF[3 * i + j][1]);
-                dR[3 * i + j][0] = fmaf(ta[j], eR[i][0], dR[3 * i + j][0]);
-                dR[3 * i + j][1] = fmaf(ta[j], eR[i][1], dR[3 * i + j][1]);
-            }
-            if (kSource) {
-                sF[i][0] = fmaf(ta[i], gF[0], sF[i][0]);
-                sF[i][1] = fmaf(ta[i], gF[1], sF[i][1]);
-                sR[i][0] = fmaf(wa, gR[i][0], sR[i][0]);
-                sR[i][1] = fmaf(wa, gR[i][1], sR[i][1]);
+                const float wj = j == corner ? w.wc[g] : w.wb[g];
+                e[j][0] = fmaf(re, wj, e[j][0]);
+                e[j][1] = fmaf(im, wj, e[j][1]);
             }
         }
     }
+    // += f times another sum
+    __device__ __forceinline__ void add_scaled(float f, const BasisSum &o) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            if constexpr (kShared) s[c] = fmaf(f, o.s[c], s[c]);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) e[j][c] = fmaf(f, o.e[j][c], e[j][c]);
+        }
+    }
+    __device__ __forceinline__ float sum(int j, int c) const {
+        return kShared ? s[c] + e[j][c] : e[j][c];
+    }
+};
+
+// a flipped in sign where bit c of the mask is set (uniform: scalar unit)
+__device__ __forceinline__ float flip(float a, int mask, int c) {
+    return __int_as_float(__float_as_int(a) ^ (((mask >> c) & 1) << 31));
 }
 
 // The fields of a test triangle's records the regular kernel uses.  They are
@@ -257,11 +233,9 @@ __device__ __forceinline__ void regular_both(const XT (&xa_m)[18], const float (
 // v_readlane, so waiting for them never waits for the LDS adds in flight
 // (scalar loads share their counter with LDS operations).
 struct TestRec {
-    float x[18];   // quadrature points
+    float xo[18];  // quadrature points as offsets from vertex 0
     float n[3];    // unit normal
     float v0[3];   // vertex 0
-    float e1[3];   // v1 - v0
-    float e2[3];   // v2 - v0
     float jac;     // 2 * area
     int vid[3];    // vertex ids
     int key[3];    // coordinate-key ids under the identity
@@ -284,13 +258,11 @@ __device__ __forceinline__ void unpack_test(int w, TestRec &r) {
     auto f = [w](int j) { return __int_as_float(__builtin_amdgcn_readlane(w, j)); };
     auto i = [w](int j) { return __builtin_amdgcn_readlane(w, 32 + j); };
 #pragma unroll
-    for (int j = 0; j < 18; ++j) r.x[j] = f(j);
+    for (int j = 0; j < 18; ++j) r.xo[j] = f(j);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         r.n[c] = f(18 + c);
         r.v0[c] = f(23 + c);
-        r.e1[c] = f(26 + c) - r.v0[c];
-        r.e2[c] = f(29 + c) - r.v0[c];
         r.dof[c] = i(c);
         r.vid[c] = i(3 + c);
         r.key[c] = i(6 + c);
@@ -301,217 +273,179 @@ __device__ __forceinline__ void unpack_test(int w, TestRec &r) {
     r.dev = i(23);
 }
 
-// All images of one (t, s): tr is t's record (uniform), yp / v0s / ns the
-// lane's points, vertex 0 and normal; rf (0 or 1) keeps or drops the (s, t)
-// double-layer block.
+// One (t, s) over all images and both directions: tr is t's record (uniform),
+// yo / v0s / ns the lane's trial points (offsets from vertex 0), vertex 0 and
+// normal.  Adds jac_t times the block sums over the 6 x 6 rule to
+//   dF[c][j][i] (test basis i on t, trial basis j on s),
+//   dR[c][i][j] (test basis i on s, trial basis j on t), c = re, im,
+// as -4 pi DLP / jac_s; sF[c][i] (basis on t) and sR[i][c] (basis on s) get
+// 4 pi SLP / (jac_s jac_t) with unit source density.  Bit m of skip drops
+// image m for the lane, rf = 0 the (s, t) double-layer block.
+//
+// Distances: d = y_b - S_m x_a = (v0_s - S_m v0_t - S_m xo_a) + yo_b, every
+// difference rounded relative to its own size (the vertices are exact floats),
+// in FP64 with kPrecise, where the phase is formed in FP64 too.  Both triangles
+// are flat, so the normal projections of d depend on one point only:
+//   d . n_s       = (v0_s - S_m x_a) . n_s    = hF[a]
+//   d . (S_m n_t) = (y_b - S_m v0_t) . (S_m n_t) = hR[b]
+// Only non-touching combinations count, so r > 0; a skipped lane's triangle is
+// moved 1000 m away, which keeps it finite, and its factors are zero.
+//
+// Loop order: test points outer, images inner, trial points innermost, so the
+// sums over t's basis weights are formed once per test point for all images,
+// and hF multiplies an image's sums once.
 template <bool kComplexK, bool kSource, int kM, bool kPrecise>
-__device__ __forceinline__ void regular_images(const TestRec &tr, int n_masks,
-                                               int packed_masks, unsigned skip,
-                                               const float (&yp)[18], const float (&v0s)[3],
-                                               const float (&ns)[3], float k, float krev,
-                                               double krev64, float kim, float rf,
-                                               float (&dF)[9][2],
-                                               float (&dR)[9][2], float (&sF)[3][2],
-                                               float (&sR)[3][2]) {
-    // one or two images: unrolled; four: a runtime loop (code size)
-    const int nm = kM < 4 ? kM : n_masks;
-    for (int m = 0; m < nm; ++m) {
-        if ((skip >> m) & 1u) continue;
-        const int mask = (packed_masks >> (3 * m)) & 7;
-        const float sg[3] = {(mask & 1) ? -1.0f : 1.0f, (mask & 2) ? -1.0f : 1.0f,
-                             (mask & 4) ? -1.0f : 1.0f};
-        float nt[3];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) nt[c] = sg[c] * tr.n[c];
-        using XT = typename std::conditional<kPrecise, double, float>::type;
-        XT xm[18];
-        float hF[6], hR[6];
-        if constexpr (kPrecise) {
-            double av[3];
-            float avf[3];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                av[c] = (double)v0s[c] - (double)(sg[c] * tr.v0[c]);  // exact
-                avf[c] = (float)av[c];
-            }
-#pragma unroll
-            for (int a = 0; a < 6; ++a) {
-                float h = 0.0f;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const float xo = fmaf((float)kRule6X[a], tr.e1[c], (float)kRule6Y[a] * tr.e2[c]);
-                    xm[3 * a + c] = av[c] - (double)(sg[c] * xo);
-                    h = fmaf((float)xm[3 * a + c], ns[c], h);
-                }
-                hF[a] = h;
-            }
-#pragma unroll
-            for (int bq = 0; bq < 6; ++bq) {
-                float h = 0.0f;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) h = fmaf(yp[3 * bq + c] + avf[c], nt[c], h);
-                hR[bq] = h * rf;  // rf = 0 drops the (s, t) double-layer block
-            }
-        } else {
-#pragma unroll
-            for (int a = 0; a < 6; ++a) {
-                float h = 0.0f;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    xm[3 * a + c] = sg[c] * tr.x[3 * a + c];
-                    h = fmaf(v0s[c] - xm[3 * a + c], ns[c], h);
-                }
-                hF[a] = h;
-            }
-            float v0t[3];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) v0t[c] = sg[c] * tr.v0[c];
-#pragma unroll
-            for (int bq = 0; bq < 6; ++bq) {
-                float h = 0.0f;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) h = fmaf(yp[3 * bq + c] - v0t[c], nt[c], h);
-                hR[bq] = h * rf;  // rf = 0 drops the (s, t) double-layer block
-            }
-        }
-        regular_both<kComplexK, kSource, kPrecise>(xm, hF, hR, yp, k, krev, krev64, kim, tr.jac,
-                                                   dF, dR, sF, sR);
-    }
-}
-
-// FP32 path of one (t, s) over all images with the test points outer and
-// the images inner: the image sums of a test point share one outer product
-// with t's basis weights (dF / dR / sF / sR are linear in the image sums),
-// so the 3 x 3 block accumulation costs 36 FMAs per test point instead of
-// 36 per test point and image.  hR[m][b] are formed once per pair.  The
-// kernel is issue-bound, so the per-evaluation work is kept to the terms
-// that change with the trial point: q2 = 1/r^2 is folded into the phase
-// terms (g = (sin k + cos / r) / r^2 ...), the test-side normal factor hF
-// (fixed per test point and image) multiplies the image's sums once, and the
-// RHS point sum is the sum of its three basis sums (the basis weights of a
-// point add up to its weight).  Only non-touching combinations come here
-// (touching ones are skipped or go to the singular kernel), so r > 0.
-template <bool kComplexK, bool kSource, int kM>
-__device__ __forceinline__ void regular_pair_fp32(const TestRec &tr, int n_masks, int packed_masks,
-                                                  unsigned skip, const float (&yp)[18],
-                                                  const float (&v0s)[3], const float (&ns)[3],
-                                                  float k, float krev, float kim, float rf,
-                                                  float (&dF)[9][2], float (&dR)[9][2],
-                                                  float (&sF)[3][2], float (&sR)[3][2]) {
-    const int nm = kM < 4 ? kM : n_masks;
-    float sg[kM][3], hR[kM][6];
+__device__ __forceinline__ void regular_pair(const TestRec &tr, int packed_masks, unsigned skip,
+                                             const RuleWeights &w, const float (&yo)[18],
+                                             const float (&v0s)[3], const float (&ns)[3], float k,
+                                             float krev, double krev64, float kim, float rf,
+                                             float (&dF)[2][3][3], float (&dR)[2][3][3],
+                                             float (&sF)[3][2], float (&sR)[3][2]) {
+    using DT = typename std::conditional<kPrecise, double, float>::type;
+    DT dv[kM][3];
+    float hR[kM][6], on[kM];
 #pragma unroll
     for (int m = 0; m < kM; ++m) {
         const int mask = (packed_masks >> (3 * m)) & 7;
-        sg[m][0] = (mask & 1) ? -1.0f : 1.0f;
-        sg[m][1] = (mask & 2) ? -1.0f : 1.0f;
-        sg[m][2] = (mask & 4) ? -1.0f : 1.0f;
-        float nt[3], v0t[3];
+        on[m] = ((skip >> m) & 1u) ? 0.0f : 1.0f;
+        float nt[3], dvf[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            nt[c] = sg[m][c] * tr.n[c];
-            v0t[c] = sg[m][c] * tr.v0[c];
+            nt[c] = flip(tr.n[c], mask, c);
+            dv[m][c] = (DT)v0s[c] - (DT)flip(tr.v0[c], mask, c);
+            if (c == 0 && on[m] == 0.0f) dv[m][c] = (DT)1.0e3f;
+            dvf[c] = (float)dv[m][c];
         }
+        const float cR = -on[m] * rf * tr.jac;
 #pragma unroll
         for (int bq = 0; bq < 6; ++bq) {
-            float h = 0.0f;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) h = fmaf(yp[3 * bq + c] - v0t[c], nt[c], h);
-            hR[m][bq] = -h * rf;  // rf = 0 drops the (s, t) double-layer block
+            const float h = fmaf(yo[3 * bq] + dvf[0], nt[0],
+                                 fmaf(yo[3 * bq + 1] + dvf[1], nt[1],
+                                      (yo[3 * bq + 2] + dvf[2]) * nt[2]));
+            hR[m][bq] = h * cR;
         }
     }
+    float tF[2][3], tR[2][3];  // sums over the test points shared by t's bases
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) tF[c][j] = tR[c][j] = 0.0f;
 #pragma unroll
     for (int a = 0; a < 6; ++a) {
-        float eF[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
-        float eR[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
-        float gR[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
+        BasisSum<!kPrecise> eF, eR, gR;
+        eF.clear();
+        eR.clear();
+        gR.clear();
 #pragma unroll
         for (int m = 0; m < kM; ++m) {
-            if (m >= nm || ((skip >> m) & 1u)) continue;
-            const float xa = sg[m][0] * tr.x[3 * a], ya = sg[m][1] * tr.x[3 * a + 1],
-                        za = sg[m][2] * tr.x[3 * a + 2];
-            const float hF = fmaf(v0s[0] - xa, ns[0], fmaf(v0s[1] - ya, ns[1], (v0s[2] - za) * ns[2]));
-            float em[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};  // this image's sums before hF
+            const int mask = (packed_masks >> (3 * m)) & 7;
+            DT D[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) D[c] = dv[m][c] - (DT)flip(tr.xo[3 * a + c], mask, c);
+            const float hF =
+                fmaf((float)D[0], ns[0], fmaf((float)D[1], ns[1], (float)D[2] * ns[2])) *
+                (on[m] * tr.jac);
+            BasisSum<!kPrecise> em;  // this image's sums before hF
+            em.clear();
+// distances of the six points, then their transcendentals as one
+            // run at raised wave priority (below), then the sums
+            DT r2d[6];
+            float rinv[6], rr[6], sn[6], cs[6];
 #pragma unroll
             for (int bq = 0; bq < 6; ++bq) {
-                const float dx = yp[3 * bq] - xa;
-                const float dy = yp[3 * bq + 1] - ya;
-                const float dz = yp[3 * bq + 2] - za;
-                const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                const float rinv = __builtin_amdgcn_rsqf(r2);
-                const float r = r2 * rinv;
-                const float t = __builtin_amdgcn_fractf(r * krev);  // revolutions, [0, 1)
-                const float sn = __builtin_amdgcn_sinf(t);
-                const float cs = __builtin_amdgcn_cosf(t);
-                float q2 = rinv * rinv;
-                float damp = 1.0f;
-                if (kComplexK) {
-                    damp = __expf(-kim * r);
-                    q2 *= damp;
+                const DT dx = D[0] + (DT)yo[3 * bq];
+                const DT dy = D[1] + (DT)yo[3 * bq + 1];
+                const DT dz = D[2] + (DT)yo[3 * bq + 2];
+                r2d[bq] = fma(dx, dx, fma(dy, dy, dz * dz));
+            }
+            trans_begin();
+#pragma unroll
+            for (int bq = 0; bq < 6; ++bq) rinv[bq] = __builtin_amdgcn_rsqf((float)r2d[bq]);
+#pragma unroll
+            for (int bq = 0; bq < 6; ++bq) {
+                const float r2 = (float)r2d[bq];
+                const float r = r2 * rinv[bq];
+                if (kComplexK) rr[bq] = r;
+                float t;  // revolutions
+                if constexpr (kPrecise) {
+                    const double rd =
+                        (double)r + fma(-(double)r, (double)r, r2d[bq]) * (double)(0.5f * rinv[bq]);
+                    double td = rd * krev64;
+                    td -= rint(td);
+                    t = (float)td;
+                } else {
+                    t = __builtin_amdgcn_fractf(r * krev);
                 }
-                const float fr = kComplexK ? rinv + kim : rinv;
-                // g = p q2 with p1 = sin k + cos fr, p2 = sin fr - cos k
-                const float kq = k * q2, fq = fr * q2;
-                const float g1 = fmaf(sn, kq, cs * fq);
-                const float g2 = fmaf(-cs, kq, sn * fq);
-                const float r1 = g1 * hR[m][bq], r2v = g2 * hR[m][bq];
-                const float wb = (float)kRule6W[bq];
-                const float w1 = wb * (float)kRule6X[bq];
-                const float w2 = wb * (float)kRule6Y[bq];
-                const float w0 = wb - w1 - w2;
-                em[0][0] = fmaf(g1, w0, em[0][0]);
-                em[0][1] = fmaf(g2, w0, em[0][1]);
-                em[1][0] = fmaf(g1, w1, em[1][0]);
-                em[1][1] = fmaf(g2, w1, em[1][1]);
-                em[2][0] = fmaf(g1, w2, em[2][0]);
-                em[2][1] = fmaf(g2, w2, em[2][1]);
-                eR[0][0] = fmaf(r1, w0, eR[0][0]);
-                eR[0][1] = fmaf(r2v, w0, eR[0][1]);
-                eR[1][0] = fmaf(r1, w1, eR[1][0]);
-                eR[1][1] = fmaf(r2v, w1, eR[1][1]);
-                eR[2][0] = fmaf(r1, w2, eR[2][0]);
-                eR[2][1] = fmaf(r2v, w2, eR[2][1]);
+                sn[bq] = t;
+            }
+#pragma unroll
+            for (int bq = 0; bq < 6; ++bq) {
+                cs[bq] = __builtin_amdgcn_cosf(sn[bq]);
+                sn[bq] = __builtin_amdgcn_sinf(sn[bq]);
+                if (kComplexK) rr[bq] = __expf(-kim * rr[bq]);  // damping
+            }
+            trans_end();
+#pragma unroll
+            for (int bq = 0; bq < 6; ++bq) {
+                float q2 = rinv[bq] * rinv[bq];
+                const float damp = kComplexK ? rr[bq] : 1.0f;
+                if (kComplexK) q2 *= damp;
+                const float fr = kComplexK ? rinv[bq] + kim : rinv[bq];
+                // -4 pi dG/dn = proj/r^2 * (cos fr + sin k, sin fr - cos k) e^{-kim r}
+                const float g1 = fmaf(sn[bq], k, cs[bq] * fr) * q2;
+                const float g2 = fmaf(-cs[bq], k, sn[bq] * fr) * q2;
+                em.add(w, bq, g1, g2);
+                eR.add(w, bq, g1 * hR[m][bq], g2 * hR[m][bq]);
                 if (kSource) {
-                    const float gv = rinv * damp;
-                    const float gc = cs * gv, gs = sn * gv;
-                    gR[0][0] = fmaf(gc, w0, gR[0][0]);
-                    gR[0][1] = fmaf(gs, w0, gR[0][1]);
-                    gR[1][0] = fmaf(gc, w1, gR[1][0]);
-                    gR[1][1] = fmaf(gs, w1, gR[1][1]);
-                    gR[2][0] = fmaf(gc, w2, gR[2][0]);
-                    gR[2][1] = fmaf(gs, w2, gR[2][1]);
+                    const float gv = rinv[bq] * damp * on[m];
+                    gR.add(w, bq, cs[bq] * gv, sn[bq] * gv);
                 }
             }
+            eF.add_scaled(hF, em);
+        }
+        const int ga = kRule6Group[a], ca = kRule6Corner[a];
+        const float wb = w.wb[ga], wa = w.wa[ga], wc = w.wc[ga];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
-                eF[j][0] = fmaf(hF, em[j][0], eF[j][0]);
-                eF[j][1] = fmaf(hF, em[j][1], eF[j][1]);
-            }
-        }
-        const float wa = (float)kRule6W[a] * tr.jac;
-        const float ta[3] = {wa * (float)(1.0 - kRule6X[a] - kRule6Y[a]), wa * (float)kRule6X[a],
-                             wa * (float)kRule6Y[a]};
-        float gF[2] = {0.f, 0.f};
-        if (kSource) {
-            gF[0] = gR[0][0] + gR[1][0] + gR[2][0];
-            gF[1] = gR[0][1] + gR[1][1] + gR[2][1];
-        }
+                const float f = eF.sum(j, c), r = eR.sum(j, c);
+                if constexpr (kPrecise) {
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                dF[3 * i + j][0] = fmaf(ta[i], eF[j][0], dF[3 * i + j][0]);
-                dF[3 * i + j][1] = fmaf(ta[i], eF[j][1], dF[3 * i + j][1]);
-                dR[3 * i + j][0] = fmaf(ta[j], eR[i][0], dR[3 * i + j][0]);
-                dR[3 * i + j][1] = fmaf(ta[j], eR[i][1], dR[3 * i + j][1]);
+                    for (int i = 0; i < 3; ++i) {
+                        dF[c][j][i] = fmaf(i == ca ? wc : wb, f, dF[c][j][i]);
+                        dR[c][j][i] = fmaf(i == ca ? wc : wb, r, dR[c][j][i]);
+                    }
+                } else {
+                    tF[c][j] = fmaf(wb, f, tF[c][j]);
+                    dF[c][j][ca] = fmaf(wa, f, dF[c][j][ca]);
+                    tR[c][j] = fmaf(wb, r, tR[c][j]);
+                    dR[c][j][ca] = fmaf(wa, r, dR[c][j][ca]);
+                }
             }
             if (kSource) {
-                sF[i][0] = fmaf(ta[i], gF[0], sF[i][0]);
-                sF[i][1] = fmaf(ta[i], gF[1], sF[i][1]);
-                sR[i][0] = fmaf(wa, gR[i][0], sR[i][0]);
-                sR[i][1] = fmaf(wa, gR[i][1], sR[i][1]);
+                const float g0 = gR.sum(0, c), g1 = gR.sum(1, c), g2 = gR.sum(2, c);
+                const float gF = g0 + g1 + g2;
+                const float wt = (float)kRule6W[a];
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    sF[i][c] = fmaf((float)(kRule6W[a] * rule6_phi(a, i)), gF, sF[i][c]);
+                sR[0][c] = fmaf(wt, g0, sR[0][c]);
+                sR[1][c] = fmaf(wt, g1, sR[1][c]);
+                sR[2][c] = fmaf(wt, g2, sR[2][c]);
             }
         }
+    }
+    if constexpr (!kPrecise) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    dF[c][j][i] += tF[c][j];
+                    dR[c][j][i] += tR[c][j];
+                }
     }
 }
 
@@ -548,38 +482,33 @@ __device__ __forceinline__ void regular_tile_pair(
     if constexpr (!kGather)
         for (int e = threadIdx.x; e < 4 * snd * tnd; e += 256) acc[e] = 0.0f;
 
-    const float k = k_real[b];
-    const float kim = kComplexK ? k_imag[b] : 0.0f;
-    const float krev = k * kInv2Pi;
+    const float k = in_vgpr(k_real[b]);
+    const float kim = kComplexK ? in_vgpr(k_imag[b]) : 0.0f;
+    const float krev = in_vgpr(k * kInv2Pi);
     const double krev64 = (double)k * kInv2PiD;
     constexpr int M = kM;  // 1 + image masks (the session's n_masks)
     const int packed_masks = g.masks[0] | (g.masks[1] << 3) | (g.masks[2] << 6) | (g.masks[3] << 9);
 
     const bool trial_ok = lane < scount;
     const int tr = s0 + (trial_ok ? lane : 0);
-    // the lane's points: absolute, or (kPrecise) offsets from vertex 0
-    float yp[18], ns[3], v0s[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        ns[c] = g.tri_f_soa[(size_t)(18 + c) * T + tr];
-        v0s[c] = g.tri_f_soa[(size_t)(23 + c) * T + tr];
-    }
-    if constexpr (kPrecise) {
+    // the lane's points as offsets from vertex 0
+    float yo[18], ns[3], v0s[3];
+    {
         float e1[3], e2[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
+            ns[c] = g.tri_f_soa[(size_t)(18 + c) * T + tr];
+            v0s[c] = g.tri_f_soa[(size_t)(23 + c) * T + tr];
             e1[c] = g.tri_f_soa[(size_t)(26 + c) * T + tr] - v0s[c];
             e2[c] = g.tri_f_soa[(size_t)(29 + c) * T + tr] - v0s[c];
         }
 #pragma unroll
-        for (int b = 0; b < 6; ++b)
+        for (int bq = 0; bq < 6; ++bq)
 #pragma unroll
             for (int c = 0; c < 3; ++c)
-                yp[3 * b + c] = fmaf((float)kRule6X[b], e1[c], (float)kRule6Y[b] * e2[c]);
-    } else {
-#pragma unroll
-        for (int j = 0; j < 18; ++j) yp[j] = g.tri_f_soa[(size_t)j * T + tr];
+                yo[3 * bq + c] = fmaf((float)kRule6X[bq], e1[c], (float)kRule6Y[bq] * e2[c]);
     }
+    const RuleWeights weights = rule_weights();
     const float jac_s = g.tri_f_soa[(size_t)22 * T + tr];
     int svid[3], skid[kMaxMasks][3], slc[3], sdof[3];
 #pragma unroll
@@ -688,13 +617,17 @@ __device__ __forceinline__ void regular_tile_pair(
         }
     }
     const unsigned long long tq_mask = __ballot(tq_lane);
-    // dF[3 r + j] / dR[3 i + r]: sums for the dof at local position r of the
+    // dF[c][j][r] / dR[c][i][r]: sums for the dof at local position r of the
     // current test, kept across tests while that position's dof is
     // unchanged (the test-side records keep shared dofs in place), and added
     // to the LDS tables only when it changes and after the last test.
-    float dF[9][2], dR[9][2];
+    float dF[2][3][3], dR[2][3][3];
 #pragma unroll
-    for (int i = 0; i < 9; ++i) dF[i][0] = dF[i][1] = dR[i][0] = dR[i][1] = 0.0f;
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int r = 0; r < 3; ++r) dF[c][i][r] = dR[c][i][r] = 0.0f;
     int held[3] = {-1, -1, -1};  // tile dof slot of each position
     auto flush = [&](int r) {
         if (kGather && gather) {
@@ -705,10 +638,10 @@ __device__ __forceinline__ void regular_tile_pair(
             float v[3][4];
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
-                v[j][0] = trial_ok ? dF[3 * r + j][0] * dscale : 0.0f;
-                v[j][1] = trial_ok ? dF[3 * r + j][1] * dscale : 0.0f;
-                v[j][2] = trial_ok ? dR[3 * j + r][0] * dscale : 0.0f;
-                v[j][3] = trial_ok ? dR[3 * j + r][1] * dscale : 0.0f;
+                v[j][0] = trial_ok ? dF[0][j][r] * dscale : 0.0f;
+                v[j][1] = trial_ok ? dF[1][j][r] * dscale : 0.0f;
+                v[j][2] = trial_ok ? dR[0][j][r] * dscale : 0.0f;
+                v[j][3] = trial_ok ? dR[1][j][r] * dscale : 0.0f;
             }
             const int nh = snd > 64 ? 2 : 1;
 #pragma unroll
@@ -745,19 +678,19 @@ __device__ __forceinline__ void regular_tile_pair(
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 // LDS table adds: relaxed, workgroup scope (no ordering among them)
-                __hip_atomic_fetch_add(cF + slc[j], dF[3 * r + j][0] * dscale, __ATOMIC_RELAXED,
+                __hip_atomic_fetch_add(cF + slc[j], dF[0][j][r] * dscale, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(cF + slc[j] + plane, dF[3 * r + j][1] * dscale,
+                __hip_atomic_fetch_add(cF + slc[j] + plane, dF[1][j][r] * dscale,
                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(cR + slc[j], dR[3 * j + r][0] * dscale, __ATOMIC_RELAXED,
+                __hip_atomic_fetch_add(cR + slc[j], dR[0][j][r] * dscale, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(cR + slc[j] + plane, dR[3 * j + r][1] * dscale,
+                __hip_atomic_fetch_add(cR + slc[j] + plane, dR[1][j][r] * dscale,
                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
         }
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-            dF[3 * r + j][0] = dF[3 * r + j][1] = dR[3 * j + r][0] = dR[3 * j + r][1] = 0.0f;
+            dF[0][j][r] = dF[1][j][r] = dR[0][j][r] = dR[1][j][r] = 0.0f;
     };
     int rec = 0;
     if (n_tests > 0)
@@ -799,60 +732,51 @@ __device__ __forceinline__ void regular_tile_pair(
                     touch |= (m == 0) ? (cur.vid[i] == svid[j]) : (cur.key[i] == skid[m][j]);
             if (m < M && touch) skip |= 1u << m;
         }
-        float sF[3][2], sR[3][2];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) sF[i][0] = sF[i][1] = sR[i][0] = sR[i][1] = 0.0f;
+        float sF[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
+        float sR[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
         const float rf = rev ? 1.0f : 0.0f;
         const bool src = wave_has_source || test_source;
-        if constexpr (kPrecise) {
-            if (src)
-                regular_images<kComplexK, true, kM, true>(cur, g.n_masks, packed_masks, skip, yp,
-                                                          v0s, ns, k, krev, krev64, kim, rf, dF,
-                                                          dR, sF, sR);
-            else
-                regular_images<kComplexK, false, kM, true>(cur, g.n_masks, packed_masks, skip, yp,
-                                                           v0s, ns, k, krev, krev64, kim, rf, dF,
-                                                           dR, sF, sR);
-        } else {
-            if (src)
-                regular_pair_fp32<kComplexK, true, kM>(cur, g.n_masks, packed_masks, skip, yp, v0s,
-                                                       ns, k, krev, kim, rf, dF, dR, sF, sR);
-            else
-                regular_pair_fp32<kComplexK, false, kM>(cur, g.n_masks, packed_masks, skip, yp,
-                                                        v0s, ns, k, krev, kim, rf, dF, dR, sF, sR);
-        }
+        if (src)
+            regular_pair<kComplexK, true, kM, kPrecise>(cur, packed_masks, skip, weights, yo, v0s,
+                                                        ns, k, krev, krev64, kim, rf, dF, dR, sF,
+                                                        sR);
+        else
+            regular_pair<kComplexK, false, kM, kPrecise>(cur, packed_masks, skip, weights, yo, v0s,
+                                                         ns, k, krev, krev64, kim, rf, dF, dR, sF,
+                                                         sR);
         if (src) {
             // Robin fold in the units of dF / dR (scaled by dscale when they
             // reach the tables): -(i k beta / 3) SLP = dscale * (+(i k beta / 3) s)
             if (lane_robin) {
+                const float cre = cFre * cur.jac, cim = cFim * cur.jac;
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
-                    const float are = cFre * sF[i][0] - cFim * sF[i][1];
-                    const float aim = cFre * sF[i][1] + cFim * sF[i][0];
+                    const float are = cre * sF[i][0] - cim * sF[i][1];
+                    const float aim = cre * sF[i][1] + cim * sF[i][0];
 #pragma unroll
                     for (int j = 0; j < 3; ++j) {
-                        dF[3 * i + j][0] += are;
-                        dF[3 * i + j][1] += aim;
+                        dF[0][j][i] += are;
+                        dF[1][j][i] += aim;
                     }
                 }
             }
             if (test_robin && rev) {
-                const float cRre = (-kim * tbre - k * tbim) * (1.0f / 3.0f);
-                const float cRim = (-kim * tbim + k * tbre) * (1.0f / 3.0f);
+                const float cRre = (-kim * tbre - k * tbim) * (1.0f / 3.0f) * cur.jac;
+                const float cRim = (-kim * tbim + k * tbre) * (1.0f / 3.0f) * cur.jac;
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
                     const float are = cRre * sR[i][0] - cRim * sR[i][1];
                     const float aim = cRre * sR[i][1] + cRim * sR[i][0];
 #pragma unroll
                     for (int j = 0; j < 3; ++j) {
-                        dR[3 * i + j][0] += are;
-                        dR[3 * i + j][1] += aim;
+                        dR[0][i][j] += are;
+                        dR[1][i][j] += aim;
                     }
                 }
             }
         }
         if (src) {
-            const float gsc = gscale;  // sF / sR carry 2 area(t)
+            const float gsc = gscale * cur.jac;  // sF / sR carry no Jacobian
             for (int sv = 0; sv < n_src; ++sv) {
                 float *rb = rhs + ((size_t)b * n_src + sv) * rhs_stride * 2;
                 const size_t lq = (((size_t)b * n_src + sv) * T + orig) * 2;

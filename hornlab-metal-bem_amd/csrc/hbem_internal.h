@@ -81,7 +81,8 @@ struct Plan {
     // position t0 + 16 w + i of a tile holds the i-th test of wave w, the
     // wave's tests ordered as a path through shared edges, each record's
     // vertices permuted so that a dof shared with the previous test keeps
-    // its local position; int word 23 is the test's device index.
+    // its local position; int word 23 is the test's device index, float words
+    // 0..17 are the quadrature points as offsets from the record's vertex 0.
     std::vector<float> tri_t_f;
     std::vector<int32_t> tri_t_i;
 

@@ -581,6 +581,13 @@ std::string build_plan(int nv, int T, int n, int symmetry, const float *vtx, con
                             }
                     const size_t q = static_cast<size_t>(base + k);
                     fill_record(p, o, &P->tri_t_f[q * kTriF], &P->tri_t_i[q * kTriI]);
+                    float *tf = &P->tri_t_f[q * kTriF];
+                    for (int a = 0; a < 6; ++a)
+                        for (int c = 0; c < 3; ++c) {
+                            const double v0 = tf[23 + c];
+                            tf[3 * a + c] = static_cast<float>(kRule6X[a] * (tf[26 + c] - v0) +
+                                                               kRule6Y[a] * (tf[29 + c] - v0));
+                        }
                     P->tri_t_i[q * kTriI + 23] = p;
                     for (int r = 0; r < 3; ++r) held[r] = slot(p, o[r]);
                 }
