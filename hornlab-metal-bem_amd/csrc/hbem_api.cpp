@@ -141,7 +141,7 @@ struct hbem_session {
     hipStream_t stream = nullptr;
     hbem::Plan plan;
     hbem::DeviceGeometry dg{};
-    DevBuf tri_f_aos, tri_i_aos, tri_t_f, tri_t_i, tri_f_soa, tri_i_soa, sg_f, sg_i, sg_rule, sg_rule_reg, tile_start,
+    DevBuf tri_f_aos, tri_i_aos, tri_t_f, tri_t_i, tri_f_soa, tri_i_soa, sg_f, sg_i, sg_rule, sg_rule_reg, gather, tile_groups, row_map, tile_touch, tile_start,
         tile_count, tile_ndofs, tile_dofs, tile_pairs, nc_f, nc_i, nc_rule, sg_adj, vtx_d, triv_d,
         normals_d, jac_d;
     // CHIEF rows and solves of the current resident batch
@@ -184,7 +184,7 @@ struct hbem_session {
 
     ~hbem_session() {
         for (DevBuf *b : {&tri_f_aos, &tri_i_aos, &tri_t_f, &tri_t_i, &tri_f_soa, &tri_i_soa, &sg_f, &sg_i,
-                          &sg_rule, &sg_rule_reg, &tile_start, &tile_count, &tile_ndofs, &tile_dofs, &tile_pairs, &nc_f, &nc_i, &nc_rule, &sg_adj, &vtx_d, &triv_d, &normals_d, &jac_d, &adj_k, &adj_kim, &adj_fk, &adj_q, &adj_beta, &adj_obs, &adj_c, &adj_ft, &adj_sig, &adj_gN, &adj_l32, &adj_e64, &adj_l64, &adj_r64, &adj_act, &chief_C, &chief_d, &chief_pts, &chief_z, &chief_e, &chief_z64, &chief_r, &chief_ainf, &A, &A_orig, &rhs, &x, &x64, &r64, &xprev, &ipiv, &info, &gl, &lu_scr_i, &lu_scr_f, &lu_pack, &amax, &lu_scale, &kv, &kh, &kn, &kf, &q, &kre,
+                          &sg_rule, &sg_rule_reg, &gather, &tile_groups, &row_map, &tile_touch, &tile_start, &tile_count, &tile_ndofs, &tile_dofs, &tile_pairs, &nc_f, &nc_i, &nc_rule, &sg_adj, &vtx_d, &triv_d, &normals_d, &jac_d, &adj_k, &adj_kim, &adj_fk, &adj_q, &adj_beta, &adj_obs, &adj_c, &adj_ft, &adj_sig, &adj_gN, &adj_l32, &adj_e64, &adj_l64, &adj_r64, &adj_act, &chief_C, &chief_d, &chief_pts, &chief_z, &chief_e, &chief_z64, &chief_r, &chief_ainf, &A, &A_orig, &rhs, &x, &x64, &r64, &xprev, &ipiv, &info, &gl, &lu_scr_i, &lu_scr_f, &lu_pack, &amax, &lu_scale, &kv, &kh, &kn, &kf, &q, &kre,
                           &kim, &fk, &obs, &field, &tags, &tagout, &norms, &anorm, &active,
                           &rowsplit, &rcx, &rcy, &rc_state, &rc_est, &io_k, &io_kim, &io_fk, &io_q, &io_obs, &io_field,
                           &io_p, &io_tag, &io_beta, &qt, &l2g, &lu_perm, &lu_pi, &lu_lf, &lu_dinv, &ts_ctx[0],
@@ -435,6 +435,10 @@ int32_t hbem_session_create(const hbem_geometry *geom, hbem_session **out) {
         upload(s->sg_i, P.sg_i, s->stream);
         upload(s->sg_rule, P.sg_rule, s->stream);
         upload(s->sg_rule_reg, P.sg_rule_reg, s->stream);
+        upload(s->gather, P.gather, s->stream);
+        upload(s->tile_groups, P.tile_groups, s->stream);
+        upload(s->row_map, P.row_map, s->stream);
+        upload(s->tile_touch, P.tile_touch, s->stream);
         upload(s->tile_start, P.tile_start, s->stream);
         upload(s->tile_count, P.tile_count, s->stream);
         upload(s->tile_ndofs, P.tile_ndofs, s->stream);
@@ -488,6 +492,12 @@ int32_t hbem_session_create(const hbem_geometry *geom, hbem_session **out) {
         g.n_tile_pairs = (int)(P.tile_pairs.size() / 2);
         g.n_tiles = (int)P.tile_start.size();
         g.max_tile_dofs = P.max_tile_dofs;
+        g.gather = s->gather.as<uint32_t>();
+        g.tile_groups = s->tile_groups.as<int32_t>();
+        g.row_map = s->row_map.as<uint32_t>();
+        g.tile_touch = s->tile_touch.as<int32_t>();
+        g.gather_groups = P.gather_groups;
+        g.run_rows = P.run_rows;
         hip_check(hipStreamSynchronize(s->stream), "session upload");
         s->setup_seconds = now_s() - t0;
         *out = s.release();

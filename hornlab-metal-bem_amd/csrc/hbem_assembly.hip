@@ -111,19 +111,27 @@ __device__ __forceinline__ GD kernel_gd_far(double dx, double dy, double dz, flo
 // Regular pairs.
 // One block = one unordered pair {T, S} of tiles of up to 64 triangles, for
 // one frequency (grid.y).  Lanes own the triangles s of S (records in
-// registers); each wave walks 16 triangles t of T, whose records are
-// wave-uniform (scalar loads).  The quadrature kernel is reciprocal: for an
-// image mask m the point sets of (test t, trial s^m) and (test s, trial t^m)
-// are isometric, |S_m y_b - x_a| = |y_b - S_m x_a|, so one evaluation of
-// r, 1/r, sin and cos at (a, b) serves both blocks:
+// registers); each wave walks a run of 16 triangles t of T, whose records are
+// wave-uniform.  The quadrature kernel is reciprocal: for an image mask m the
+// point sets of (test t, trial s^m) and (test s, trial t^m) are isometric,
+// |S_m y_b - x_a| = |y_b - S_m x_a|, so one evaluation of r, 1/r, sin and cos
+// at (a, b) serves both blocks:
 //   (t, s^m):  d = y_b - S_m x_a,  proj =  d . n_s
 //   (s, t^m):                      proj = -d . (S_m n_t)
-// (S_m is its own inverse and orthogonal).  The two 3x3 blocks are summed in
-// two LDS images of the tiles' (rows x cols) sub-matrices with LDS float
-// atomics and leave with one global atomic add per touched entry.  On a
-// diagonal block (T == S) lane s does the pair {t, s} only for s >= t, the
-// second direction only for s > t.  Images run in a runtime loop (mirror
-// signs applied to the uniform test points).
+// (S_m is its own inverse and orthogonal).  On a diagonal block (T == S) lane
+// s does the pair {t, s} only for s >= t, the second direction only for s > t.
+//
+// Block sums.  The 3x3 blocks of a test stay in registers while the next test
+// (the runs are ordered as paths through shared edges) keeps its dofs.  When a
+// dof leaves, its row goes to the wave's LDS table [row][trial dof] of
+// (F re, F im, R re, R im): the lanes stage their three values, and the lane
+// that owns a trial dof adds up the staged values of its triangles and updates
+// the table entry with one 16-byte read and write.  The table belongs to one
+// wave, so no LDS atomics (2 cycles per lane: 1380 cycles of the CU's LDS per
+// row with twelve per trial lane, 650 when gathered first; about 170 here).
+// At the end the block adds up its waves' tables, one global atomic add per
+// touched word; a run with more dofs than table rows writes its table out
+// earlier, on its own.
 // ---------------------------------------------------------------------------
 
 constexpr int kTestsPerWave = kTileTris / 4;
@@ -165,6 +173,14 @@ __device__ __forceinline__ void trans_begin() {
 __device__ __forceinline__ void trans_end() {
     __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
+}
+
+// A pointer the compiler cannot see through: addresses formed from it inside a
+// branch stay there instead of being computed before the loop and held.
+template <class T>
+__device__ __forceinline__ T *opaque(T *p) {
+    asm volatile("" : "+s"(p));
+    return p;
 }
 
 __device__ __forceinline__ RuleWeights rule_weights() {
@@ -221,6 +237,8 @@ struct BasisSum {
     }
 };
 
+typedef float v4f __attribute__((ext_vector_type(4)));
+
 // a flipped in sign where bit c of the mask is set (uniform: scalar unit)
 __device__ __forceinline__ float flip(float a, int mask, int c) {
     return __int_as_float(__float_as_int(a) ^ (((mask >> c) & 1) << 31));
@@ -239,7 +257,8 @@ struct TestRec {
     float jac;     // 2 * area
     int vid[3];    // vertex ids
     int key[3];    // coordinate-key ids under the identity
-    int slot[3];   // tile dof slots
+    int row[3];    // rows of the wave's table
+    int seg;       // rows of a segment that ends here before the run, else 0
     int dof[3];    // P1 dofs
     int orig;      // caller index
     int dev;       // device index
@@ -266,9 +285,10 @@ __device__ __forceinline__ void unpack_test(int w, TestRec &r) {
         r.dof[c] = i(c);
         r.vid[c] = i(3 + c);
         r.key[c] = i(6 + c);
-        r.slot[c] = i(20 + c);
+        r.row[c] = i(20 + c);
     }
     r.jac = f(22);
+    r.seg = i(18);
     r.orig = i(19);
     r.dev = i(23);
 }
@@ -449,44 +469,42 @@ __device__ __forceinline__ void regular_pair(const TestRec &tr, int packed_masks
     }
 }
 
+// 16-byte words of LDS per wave: staged values and the table.
+__host__ __device__ constexpr int regular_wave_lds(int rows, int dofs) {
+    return kStageBytes / 16 + rows * dofs;
+}
+
 // One tile pair (pair index tp) at one frequency (b) of the regular
 // assembly: the block body shared by the single-mesh kernel and the
 // multi-mesh launch of a session group.
-// list entries per (trial column, local vertex) of the gathered flush
-constexpr int kGatherCap = 8;
-
 template <bool kComplexK, int kM, bool kPrecise>
 __device__ __forceinline__ void regular_tile_pair(
     const DeviceGeometry &g, int tp, int b, const float *__restrict__ k_real,
     const float *__restrict__ k_imag, const float *__restrict__ q, int n_src,
     const float *__restrict__ beta, float *__restrict__ A, int64_t lda, int64_t a_stride,
     float *__restrict__ rhs, int64_t rhs_stride) {
-    // LDS tables, each [T dofs][S dofs] with real and imaginary planes:
-    // F (rows of t, columns of s) and R (rows of s, columns of t), indexed
-    // (test slot) * snd + (trial slot), so a wave's adds for one entry hit
-    // consecutive words (one bank per distinct trial slot).
-    extern __shared__ float acc[];
+    extern __shared__ v4f regular_lds[];
     const int T = g.n_triangles;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int s_tile = g.tile_pairs[2 * tp], t_tile = g.tile_pairs[2 * tp + 1];
     const bool diag = s_tile == t_tile;
     const int s0 = g.tile_start[s_tile], scount = g.tile_count[s_tile], snd = g.tile_ndofs[s_tile];
-    const int t0 = g.tile_start[t_tile], tcount = g.tile_count[t_tile], tnd = g.tile_ndofs[t_tile];
-    const int plane = snd * tnd;
-    float *accF = acc;              // re, then im at + plane
-    float *accR = acc + 2 * plane;  // re, then im at + plane
-    // single-image FP32 blocks gather each flush per trial column (below);
-    // their tables hold the column lists first and are zeroed after
-    constexpr bool kGather = kM == 1 && !kPrecise;
-    if constexpr (!kGather)
-        for (int e = threadIdx.x; e < 4 * snd * tnd; e += 256) acc[e] = 0.0f;
+    const int t0 = g.tile_start[t_tile], tcount = g.tile_count[t_tile];
+    const int tnd = g.tile_ndofs[t_tile];
+    const int n_tests = max(0, min(kTestsPerWave, tcount - wave * kTestsPerWave));
+    // the wave's staged values [3][64] and zero slot, then its table
+    const int wave_lds = regular_wave_lds(g.run_rows, g.max_tile_dofs);
+    v4f *stage = regular_lds + wave * wave_lds;
+    v4f *table = stage + kStageBytes / 16;
+    const v4f zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (lane == 0) stage[kGatherZero] = zero4;
+    for (int e = lane; e < g.run_rows * snd; e += 64) table[e] = zero4;
 
     const float k = in_vgpr(k_real[b]);
     const float kim = kComplexK ? in_vgpr(k_imag[b]) : 0.0f;
     const float krev = in_vgpr(k * kInv2Pi);
     const double krev64 = (double)k * kInv2PiD;
-    constexpr int M = kM;  // 1 + image masks (the session's n_masks)
     const int packed_masks = g.masks[0] | (g.masks[1] << 3) | (g.masks[2] << 6) | (g.masks[3] << 9);
 
     const bool trial_ok = lane < scount;
@@ -510,19 +528,7 @@ __device__ __forceinline__ void regular_tile_pair(
     }
     const RuleWeights weights = rule_weights();
     const float jac_s = g.tri_f_soa[(size_t)22 * T + tr];
-    int svid[3], skid[kMaxMasks][3], slc[3], sdof[3];
-#pragma unroll
-    for (int l = 0; l < 3; ++l) {
-        svid[l] = g.tri_i_soa[(size_t)(3 + l) * T + tr];
-        slc[l] = g.tri_i_soa[(size_t)(20 + l) * T + tr];
-        sdof[l] = g.tri_i_soa[(size_t)l * T + tr];
-    }
-#pragma unroll
-    for (int m = 0; m < kMaxMasks; ++m)
-#pragma unroll
-        for (int l = 0; l < 3; ++l)
-            skid[m][l] = (m < M) ? g.tri_i_soa[(size_t)(6 + 3 * m + l) * T + tr] : -1;
-    (void)skid;
+    const bool touching = g.tile_touch[tp] != 0;
     const int orig = g.tri_i_soa[(size_t)19 * T + tr];
     // Neumann data of the lane's triangle for every source (q [B][S][T])
     bool lane_q = false;
@@ -542,63 +548,16 @@ __device__ __forceinline__ void regular_tile_pair(
     // -4 pi and 4 pi folded out of the kernels, jac = (2 A_test)(2 A_trial)
     const float dscale = -kInv4Pi * jac_s * g.row_weight;
     const float gscale = kInv4Pi * jac_s * g.row_weight;
-    // Column lists of the trial side (kGather): for trial dof slot c and
-    // local vertex j, the lanes whose vertex j has slot c (at most kGatherCap;
-    // more and the block keeps per-lane atomics).  A lane owns columns
-    // lane and lane + 64 and holds their lists in registers, packed one byte
-    // per entry.
-    uint32_t glist[2][3][2] = {};
-    int gcnt[2][3] = {};
-    int gmax[3] = {0, 0, 0};
-    bool gather = false;
-    if constexpr (kGather) {
-        int *cnt = reinterpret_cast<int *>(acc);                            // [3][snd]
-        unsigned char *lst = reinterpret_cast<unsigned char *>(cnt + 3 * snd);  // [3][snd][cap]
-        for (int e = threadIdx.x; e < 3 * snd; e += 256) cnt[e] = 0;
-        __syncthreads();
-        if (wave == 0 && trial_ok) {
+    // Column `lane` of the trial tile: its dof and the first words of its list
+    // of staged values.
+    const bool col_ok = lane < snd;
+    const int col_dof = g.tile_dofs[(size_t)s_tile * kGatherCols + lane];
+    const int groups = g.tile_groups[s_tile];
+    const int list_at = s_tile * g.gather_groups * kGatherCols + lane;
+    uint32_t list[kGatherHeld];
 #pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const int slot = j * snd + slc[j];
-                const int pos = atomicAdd(cnt + slot, 1);
-                if (pos < kGatherCap) lst[slot * kGatherCap + pos] = (unsigned char)lane;
-            }
-        }
-        __syncthreads();
-        int over = 0;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int c = lane + 64 * h;
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const int n = c < snd ? cnt[j * snd + c] : 0;
-                over |= n > kGatherCap;
-                gcnt[h][j] = min(n, kGatherCap);
-                if (n > 0) {
-                    const uint32_t *w = reinterpret_cast<const uint32_t *>(lst) + (j * snd + c) * 2;
-                    glist[h][j][0] = w[0];
-                    glist[h][j][1] = w[1];
-                }
-            }
-        }
-        // every lane has read the lists; the flag is block-uniform
-        gather = __syncthreads_or(over) == 0;
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            int m = max(gcnt[0][j], gcnt[1][j]);
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) m = max(m, __shfl_xor(m, off));
-            gmax[j] = __builtin_amdgcn_readfirstlane(m);
-        }
-        for (int e = threadIdx.x; e < 4 * snd * tnd; e += 256) acc[e] = 0.0f;
-    }
-    (void)glist;
-    (void)gcnt;
-    (void)gmax;
-    (void)gather;
-    __syncthreads();
+    for (int e = 0; e < kGatherHeld; ++e) list[e] = g.gather[list_at + e * kGatherCols];
 
-    const int n_tests = max(0, min(kTestsPerWave, tcount - wave * kTestsPerWave));
     // Per-test source flags and Robin admittances of this wave's tests, one
     // lane per test, read back with v_readlane inside the loop (no memory
     // access on the per-test path).
@@ -620,7 +579,7 @@ __device__ __forceinline__ void regular_tile_pair(
     // dF[c][j][r] / dR[c][i][r]: sums for the dof at local position r of the
     // current test, kept across tests while that position's dof is
     // unchanged (the test-side records keep shared dofs in place), and added
-    // to the LDS tables only when it changes and after the last test.
+    // to the table only when it changes and at the end of a segment.
     float dF[2][3][3], dR[2][3][3];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
@@ -628,69 +587,60 @@ __device__ __forceinline__ void regular_tile_pair(
         for (int i = 0; i < 3; ++i)
 #pragma unroll
             for (int r = 0; r < 3; ++r) dF[c][i][r] = dR[c][i][r] = 0.0f;
-    int held[3] = {-1, -1, -1};  // tile dof slot of each position
-    auto flush = [&](int r) {
-        if (kGather && gather) {
-            // lanes own trial columns: each sums the contributions of the
-            // lanes in its lists (cross-lane reads), then one atomic per
-            // table word and owned column
-            const int row = held[r];
-            float v[3][4];
+    int row_dof = -1;  // dof of table row `lane`
+    auto flush = [&](int r, int to_row, int dof) {
 #pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                v[j][0] = trial_ok ? dF[0][j][r] * dscale : 0.0f;
-                v[j][1] = trial_ok ? dF[1][j][r] * dscale : 0.0f;
-                v[j][2] = trial_ok ? dR[0][j][r] * dscale : 0.0f;
-                v[j][3] = trial_ok ? dR[1][j][r] * dscale : 0.0f;
-            }
-            const int nh = snd > 64 ? 2 : 1;
+        for (int j = 0; j < 3; ++j) {
+            stage[64 * j + lane] = (v4f){dF[0][j][r] * dscale, dF[1][j][r] * dscale,
+                                         dR[0][j][r] * dscale, dR[1][j][r] * dscale};
+            dF[0][j][r] = dF[1][j][r] = dR[0][j][r] = dR[1][j][r] = 0.0f;
+        }
+        if (lane == to_row) row_dof = dof;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        v4f sum = zero4;
+        auto add4 = [&](uint32_t w) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                if (h >= nh) break;
-                float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int j = 0; j < 3; ++j)
-                    for (int k = 0; k < gmax[j]; ++k) {
-                        const bool on = k < gcnt[h][j];
-                        const int src =
-                            on ? (int)((glist[h][j][k >> 2] >> (8 * (k & 3))) & 0xffu) : lane;
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const float x = __shfl(v[j][q], src);
-                            sum[q] += on ? x : 0.0f;
-                        }
-                    }
-                const int c = lane + 64 * h;
-                if (c < snd && (gcnt[h][0] + gcnt[h][1] + gcnt[h][2]) > 0) {
-                    float *cF = accF + row * snd + c;
-                    float *cR = accR + row * snd + c;
-                    __hip_atomic_fetch_add(cF, sum[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    __hip_atomic_fetch_add(cF + plane, sum[1], __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-                    __hip_atomic_fetch_add(cR, sum[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    __hip_atomic_fetch_add(cR + plane, sum[3], __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+            for (int e = 0; e < 4; ++e) sum += stage[(w >> (8 * e)) & 0xffu];
+        };
+        add4(list[0]);
+        if (groups > 1) add4(list[1]);
+        for (int e = kGatherHeld; e < groups; ++e) add4(opaque(g.gather)[list_at + e * kGatherCols]);
+        if (col_ok) table[to_row * snd + lane] += sum;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    float *Ab = A + (size_t)b * a_stride * 2;
+    auto add_to_matrix = [&](int row, int col, float re, float im) {
+        if (re != 0.0f || im != 0.0f) {
+            const size_t idx = ((size_t)col * lda + row) * 2;
+            atomicAdd(Ab + idx, re);
+            atomicAdd(Ab + idx + 1, im);
+        }
+    };
+    // a segment that ends before its run: the wave's rows to A, for F 16 rows
+    // by 4 columns per instruction, for R one row
+    auto write_table = [&](int rows) {
+        for (int r0 = 0; r0 < rows; r0 += 16) {
+            const int r = r0 + (lane & 15);
+            const int td = __shfl(row_dof, r);
+            for (int c0 = 0; c0 < snd; c0 += 4) {
+                const int c = c0 + (lane >> 4);
+                const int sd = __shfl(col_dof, c);
+                if (r < rows && c < snd) {
+                    const v4f v = table[r * snd + c];
+                    add_to_matrix(td, sd, v[0], v[1]);
                 }
             }
-        } else if (trial_ok) {
-            float *cF = accF + held[r] * snd;
-            float *cR = accR + held[r] * snd;
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                // LDS table adds: relaxed, workgroup scope (no ordering among them)
-                __hip_atomic_fetch_add(cF + slc[j], dF[0][j][r] * dscale, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(cF + slc[j] + plane, dF[1][j][r] * dscale,
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(cR + slc[j], dR[0][j][r] * dscale, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(cR + slc[j] + plane, dR[1][j][r] * dscale,
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        for (int r = 0; r < rows; ++r) {
+            const int td = __builtin_amdgcn_readlane(row_dof, r);
+            if (col_ok) {
+                const v4f v = table[r * snd + lane];
+                add_to_matrix(col_dof, td, v[2], v[3]);
+                table[r * snd + lane] = zero4;
             }
         }
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            dF[0][j][r] = dF[1][j][r] = dR[0][j][r] = dR[1][j][r] = 0.0f;
     };
     int rec = 0;
     if (n_tests > 0)
@@ -702,12 +652,6 @@ __device__ __forceinline__ void regular_tile_pair(
         const int nt_next = rbase + ti + (ti + 1 < n_tests ? 1 : 0);
         rec = rec_word(g.tri_t_f + (size_t)nt_next * kTriF, g.tri_t_i + (size_t)nt_next * kTriI,
                        lane);
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-            if (held[r] != cur.slot[r]) {
-                if (held[r] >= 0) flush(r);
-                held[r] = cur.slot[r];
-            }
         const int lt = cur.dev - t0;  // the test's position in its tile
         const int torig = cur.orig;
         const bool test_q = (tq_mask >> ti) & 1ull;
@@ -722,28 +666,42 @@ __device__ __forceinline__ void regular_tile_pair(
         // index, images by coordinate key of t against the keys of s under
         // mask m); s touches t^m exactly when t touches s^m
         unsigned skip = fwd ? 0u : 0xfu;
+        if (touching) {
+            const int32_t *ids = opaque(g.tri_i_soa);
 #pragma unroll
-        for (int m = 0; m < kM; ++m) {
-            bool touch = false;
+            for (int m = 0; m < kM; ++m) {
+                bool touch = false;
 #pragma unroll
-            for (int i = 0; i < 3; ++i)
+                for (int j = 0; j < 3; ++j) {
+                    const int id = ids[(size_t)((m == 0 ? 3 : 6 + 3 * m) + j) * T + tr];
 #pragma unroll
-                for (int j = 0; j < 3; ++j)
-                    touch |= (m == 0) ? (cur.vid[i] == svid[j]) : (cur.key[i] == skid[m][j]);
-            if (m < M && touch) skip |= 1u << m;
+                    for (int i = 0; i < 3; ++i) touch |= (m == 0 ? cur.vid[i] : cur.key[i]) == id;
+                }
+                if (touch) skip |= 1u << m;
+            }
         }
         float sF[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
         float sR[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
         const float rf = rev ? 1.0f : 0.0f;
         const bool src = wave_has_source || test_source;
-        if (src)
-            regular_pair<kComplexK, true, kM, kPrecise>(cur, packed_masks, skip, weights, yo, v0s,
-                                                        ns, k, krev, krev64, kim, rf, dF, dR, sF,
-                                                        sR);
-        else
-            regular_pair<kComplexK, false, kM, kPrecise>(cur, packed_masks, skip, weights, yo, v0s,
-                                                         ns, k, krev, krev64, kim, rf, dF, dR, sF,
-                                                         sR);
+        // images in pairs: four at once hold 24 more registers than fit
+        constexpr int kGroup = kM < 2 ? kM : 2;
+        auto images = [&](int m) {
+            if (src)
+                regular_pair<kComplexK, true, kGroup, kPrecise>(
+                    cur, packed_masks >> (3 * m), skip >> m, weights, yo, v0s, ns, k, krev, krev64,
+                    kim, rf, dF, dR, sF, sR);
+            else
+                regular_pair<kComplexK, false, kGroup, kPrecise>(
+                    cur, packed_masks >> (3 * m), skip >> m, weights, yo, v0s, ns, k, krev, krev64,
+                    kim, rf, dF, dR, sF, sR);
+        };
+        if constexpr (kM > kGroup) {
+#pragma unroll 1
+            for (int m = 0; m < kM; m += kGroup) images(m);
+        } else {
+            images(0);
+        }
         if (src) {
             // Robin fold in the units of dF / dR (scaled by dscale when they
             // reach the tables): -(i k beta / 3) SLP = dscale * (+(i k beta / 3) s)
@@ -777,10 +735,15 @@ __device__ __forceinline__ void regular_tile_pair(
         }
         if (src) {
             const float gsc = gscale * cur.jac;  // sF / sR carry no Jacobian
+            const float *q_s = opaque(q);
+            const int32_t *ids = opaque(g.tri_i_soa);
+            int sdof[3];
+#pragma unroll
+            for (int l = 0; l < 3; ++l) sdof[l] = ids[(size_t)l * T + tr];
             for (int sv = 0; sv < n_src; ++sv) {
-                float *rb = rhs + ((size_t)b * n_src + sv) * rhs_stride * 2;
+                float *rb = opaque(rhs) + ((size_t)b * n_src + sv) * rhs_stride * 2;
                 const size_t lq = (((size_t)b * n_src + sv) * T + orig) * 2;
-                const float qre = trial_ok ? q[lq] : 0.0f, qim = trial_ok ? q[lq + 1] : 0.0f;
+                const float qre = trial_ok ? q_s[lq] : 0.0f, qim = trial_ok ? q_s[lq + 1] : 0.0f;
                 if (__any(qre != 0.0f || qim != 0.0f)) {
                     // rhs_t += 2^planes SLP(t, s) q_s, reduced over the wave
 #pragma unroll
@@ -799,7 +762,7 @@ __device__ __forceinline__ void regular_tile_pair(
                     }
                 }
                 const size_t tq = (((size_t)b * n_src + sv) * T + torig) * 2;
-                const float tqre = q[tq], tqim = q[tq + 1];
+                const float tqre = q_s[tq], tqim = q_s[tq + 1];
                 if ((tqre != 0.0f || tqim != 0.0f) && rev) {
                     // rhs_s += 2^planes SLP(s, t) q_t
 #pragma unroll
@@ -810,33 +773,44 @@ __device__ __forceinline__ void regular_tile_pair(
                 }
             }
         }
-    }
+        // rows whose dof the next test does not keep in place, all at the end
+        // of a segment
+        const bool last = cur.seg > 0 || ti + 1 == n_tests;
 #pragma unroll
-    for (int r = 0; r < 3; ++r)
-        if (held[r] >= 0) flush(r);
-    __syncthreads();
-    float *Ab = A + (size_t)b * a_stride * 2;
-    const int32_t *tdofs = g.tile_dofs + (size_t)t_tile * kTileMaxDofs;
-    const int32_t *sdofs = g.tile_dofs + (size_t)s_tile * kTileMaxDofs;
-    // consecutive threads take consecutive rows of one matrix column (the
-    // atomics of a wave share cache lines)
-    for (int e = threadIdx.x; e < plane; e += 256) {
-        const int ls = e / tnd, lt_ = e - ls * tnd;
-        const float fre = accF[lt_ * snd + ls], fim = accF[lt_ * snd + ls + plane];
-        if (fre != 0.0f || fim != 0.0f) {  // A[t dof][s dof]
-            const size_t idx = ((size_t)sdofs[ls] * lda + tdofs[lt_]) * 2;
-            atomicAdd(Ab + idx, fre);
-            atomicAdd(Ab + idx + 1, fim);
-        }
+        for (int r = 0; r < 3; ++r)
+            if (last || __builtin_amdgcn_readlane(rec, 52 + r) != cur.row[r])
+                flush(r, cur.row[r], cur.dof[r]);
+        if (cur.seg > 0) write_table(cur.seg);
     }
-    for (int e = threadIdx.x; e < plane; e += 256) {
-        const int lt_ = e / snd, ls = e - lt_ * snd;
-        const float rre = accR[e], rim = accR[e + plane];
-        if (rre != 0.0f || rim != 0.0f) {  // A[s dof][t dof]
-            const size_t idx = ((size_t)tdofs[lt_] * lda + sdofs[ls]) * 2;
-            atomicAdd(Ab + idx, rre);
-            atomicAdd(Ab + idx + 1, rim);
+    __syncthreads();
+    // The sum of the four tables to A, a wave's lanes on consecutive rows of one
+    // column of A (its atomics share cache lines): for F lane = test dof and the
+    // waves share the columns, for R lane = trial dof and they share the rows.
+    const int row_dof_l = g.tile_dofs[(size_t)t_tile * kGatherCols + lane];
+    const int map_l = (int)g.row_map[(size_t)t_tile * kGatherCols + lane];
+    const int base = kStageBytes / 16;
+    auto summed = [&](int rows, int col, int half, float &re, float &im) {
+        re = im = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const int r = (rows >> (8 * w)) & 0xff;
+            const bool on = r != 0xff;
+            const v4f v = regular_lds[w * wave_lds + base + (on ? r : 0) * snd + col];
+            re += on ? v[half] : 0.0f;
+            im += on ? v[half + 1] : 0.0f;
         }
+    };
+#pragma unroll 2
+    for (int c = wave; c < snd; c += 4) {
+        float re, im;
+        summed(map_l, c, 0, re, im);
+        if (lane < tnd) add_to_matrix(row_dof_l, __builtin_amdgcn_readlane(col_dof, c), re, im);
+    }
+#pragma unroll 2
+    for (int r = wave; r < tnd; r += 4) {
+        float re, im;
+        summed(__builtin_amdgcn_readlane(map_l, r), min(lane, snd - 1), 2, re, im);
+        if (col_ok) add_to_matrix(col_dof, __builtin_amdgcn_readlane(row_dof_l, r), re, im);
     }
 }
 
@@ -1441,8 +1415,7 @@ void launch_assemble_regular(const DeviceGeometry &g, int n_batch, const float *
                              int64_t rhs_stride, hipStream_t stream, bool precise) {
     if (g.n_tile_pairs == 0 || n_batch <= 0) return;
     dim3 grid(g.n_tile_pairs, n_batch);
-    // two tables of (max tile dofs)^2 complex floats
-    const size_t shm = sizeof(float) * 4 * (size_t)g.max_tile_dofs * g.max_tile_dofs;
+    const size_t shm = 64 * (size_t)regular_wave_lds(g.run_rows, g.max_tile_dofs);
     auto go = [&](auto complex_k, auto masks) {
         constexpr bool kC = decltype(complex_k)::value;
         constexpr int kM = decltype(masks)::value;
@@ -1500,13 +1473,13 @@ void launch_assemble_multi(const AssemblyJob *jobs_dev, const std::vector<Assemb
                                  j.a_stride, j.rhs, j.rhs_stride, stream);
         return;
     }
-    int reg = 0, sing = 0, dofs = 0;
+    int reg = 0, sing = 0, words = 0;
     for (const AssemblyJob &j : jobs) {
         reg += regular_blocks(j.g, j.n_batch);
         sing += singular_blocks(j.g, j.n_batch);
-        dofs = std::max(dofs, j.g.max_tile_dofs);
+        words = std::max(words, regular_wave_lds(j.g.run_rows, j.g.max_tile_dofs));
     }
-    const size_t shm = sizeof(float) * 4 * (size_t)dofs * dofs;
+    const size_t shm = 64 * (size_t)words;
     constexpr int kFB = 2;
     auto go = [&](auto complex_k_t) {
         constexpr bool kC = decltype(complex_k_t)::value;

@@ -50,19 +50,30 @@ constexpr int kTriF = 32;
 //   [0..2]   P1 dofs
 //   [3..5]   vertex indices
 //   [6+3m .. 8+3m] coordinate-key ids of the vertices under mask index m
-//   [18]     physical tag
+//   [18]     physical tag; in test-side records the number of table rows of
+//            the segment that ends here before the run does, else 0
 //   [19]     original (caller) triangle index
-//   [20..22] position of each dof in the triangle's tile dof list
+//   [20..22] position of each dof in the triangle's tile dof list; in
+//            test-side records its row in the wave's table
 //   [23]     device index (test-side records), else -1
 constexpr int kTriI = 24;
 
 // Triangles are stored in Morton order of their centroids and grouped into
 // tiles of up to kTileTris consecutive triangles with at most kTileMaxDofs
-// distinct dofs; the regular-assembly kernel accumulates the two tile x
-// tile blocks of a tile pair in LDS (2 * 90^2 complex floats = 129600 B at
-// most).
+// distinct dofs.  A wave of the regular-assembly kernel takes a run of a test
+// tile's triangles against a whole trial tile and sums its two blocks in an LDS
+// table of its own, [rows][trial tile dofs] of (re, im, re, im); kRegularLds
+// bytes (half of a CU's LDS) bound the tables and staging areas of four waves.
+// One lane owns each trial dof.  At most 56 dofs per tile: 19 table rows fit, which nine of
+// ten runs keep to (with 64 dofs 16 rows fit and two of three runs do not),
+// and the extra tiles cost about 1%.
 constexpr int kTileTris = 64;
-constexpr int kTileMaxDofs = 90;
+constexpr int kTileMaxDofs = 56;
+constexpr int kRegularLds = 80 * 1024;
+constexpr int kGatherCols = 64;   // lanes
+constexpr int kGatherHeld = 2;    // list words per column held in registers
+constexpr int kGatherZero = 192;  // staging slot that holds zeros
+constexpr int kStageBytes = (3 * 64 + 1) * 16;  // one wave's staged values
 
 struct Plan {
     int n_vertices = 0;
@@ -169,9 +180,19 @@ struct Plan {
     std::vector<int32_t> tile_start;   // [n_tiles]
     std::vector<int32_t> tile_count;   // [n_tiles]
     std::vector<int32_t> tile_ndofs;   // [n_tiles]
-    std::vector<int32_t> tile_dofs;    // [n_tiles][kTileMaxDofs], -1 padded
+    std::vector<int32_t> tile_dofs;    // [n_tiles][kGatherCols], -1 padded
     std::vector<int32_t> tile_pairs;   // [n_tile_pairs][2] = (S, T), S >= T
     int max_tile_dofs = 0;
+    // Column lists of the trial side, [n_tiles][gather_groups][64] words of
+    // four staging slots, and the words in use per tile.
+    std::vector<uint32_t> gather;
+    std::vector<int32_t> tile_groups;  // [n_tiles]
+    int gather_groups = 0;
+    // Row of each tile dof in the last segment of the tile's four runs, a byte
+    // per run, 255 where the run does not hold it.
+    std::vector<uint32_t> row_map;  // [n_tiles][kGatherCols]
+    std::vector<int32_t> tile_touch;  // [n_tile_pairs]: some combination touches
+    int run_rows = 0;  // rows of a wave's table
 };
 
 // Builds the plan.  Returns an empty string on success, else a message.
@@ -240,6 +261,12 @@ struct DeviceGeometry {
     int n_tiles;
     int n_tile_pairs;
     int max_tile_dofs;
+    const uint32_t *gather;
+    const int32_t *tile_groups;
+    const uint32_t *row_map;
+    const int32_t *tile_touch;
+    int gather_groups;
+    int run_rows;
 };
 
 // Transcendental-pipe probe: blocks x 256 threads x iters x 16 ops

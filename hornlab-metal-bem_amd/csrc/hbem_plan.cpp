@@ -465,11 +465,43 @@ std::string build_plan(int nv, int T, int n, int symmetry, const float *vtx, con
             P->tile_start.push_back(start);
             P->tile_count.push_back(p - start);
             P->tile_ndofs.push_back((int)dofs.size());
-            dofs.resize(kTileMaxDofs, -1);
+            dofs.resize(kGatherCols, -1);
             P->tile_dofs.insert(P->tile_dofs.end(), dofs.begin(), dofs.end());
         }
         P->max_tile_dofs = *std::max_element(P->tile_ndofs.begin(), P->tile_ndofs.end());
         const int nt = static_cast<int>(P->tile_start.size());
+        // Column lists of the trial side: for column (tile dof) c the staged
+        // values 64 j + lane of the triangles whose vertex j is that dof, four
+        // bytes to a word, padded with the slot that holds zeros.
+        std::vector<std::vector<int>> lists(static_cast<size_t>(nt) * kGatherCols);
+        size_t longest = 1;
+        for (int tile = 0; tile < nt; ++tile)
+            for (int j = 0; j < 3; ++j)
+                for (int i = 0; i < P->tile_count[tile]; ++i) {
+                    const int c = ldof[3 * static_cast<size_t>(P->tile_start[tile] + i) + j];
+                    auto &l = lists[static_cast<size_t>(tile) * kGatherCols + c];
+                    l.push_back(64 * j + i);
+                    longest = std::max(longest, l.size());
+                }
+        P->gather_groups = std::max(kGatherHeld, static_cast<int>((longest + 3) / 4));
+        P->gather.assign(static_cast<size_t>(nt) * kGatherCols * P->gather_groups, 0);
+        P->tile_groups.assign(static_cast<size_t>(nt), 0);
+        for (int tile = 0; tile < nt; ++tile)
+            for (int c = 0; c < kGatherCols; ++c) {
+                const auto &l = lists[static_cast<size_t>(tile) * kGatherCols + c];
+                P->tile_groups[tile] =
+                    std::max(P->tile_groups[tile], static_cast<int>((l.size() + 3) / 4));
+                for (int g = 0; g < P->gather_groups; ++g) {
+                    uint32_t w = 0;
+                    for (int e = 0; e < 4; ++e) {
+                        const size_t k = static_cast<size_t>(4 * g + e);
+                        w |= static_cast<uint32_t>(k < l.size() ? l[k] : kGatherZero) << (8 * e);
+                    }
+                    P->gather[(static_cast<size_t>(tile) * P->gather_groups + g) * kGatherCols + c] = w;
+                }
+            }
+        P->run_rows = std::max(
+            3, static_cast<int>((kRegularLds / 4 - kStageBytes) / (16 * P->max_tile_dofs)));
         P->tile_pairs.clear();
         for (int t = 0; t < nt; ++t)
             for (int s = t; s < nt; ++s) {
@@ -516,13 +548,16 @@ std::string build_plan(int nv, int T, int n, int symmetry, const float *vtx, con
             fill_record(p, natural, &P->tri_f_aos[static_cast<size_t>(p) * kTriF],
                         &P->tri_i_aos[static_cast<size_t>(p) * kTriI]);
     }
-    // Test-side records: each wave's run of tile positions ordered as a path
-    // (the next test shares the most dofs with the current one, ties to the
-    // one with fewer unvisited edge neighbours, then the lower position), and
-    // each test's vertices placed so that dofs shared with the previous test
-    // keep their local positions.
+    // Test-side records: a tile's triangles are split into runs of 16 grown so
+    // that each adds the fewest dofs (compact patches: few table rows), each
+    // run ordered as a path (the next test shares the most dofs with the
+    // current one, ties to the one with fewer unvisited edge neighbours, then
+    // the earlier one), and each test's vertices placed so that dofs shared
+    // with the previous test keep their local positions.
     P->tri_t_f.assign(static_cast<size_t>(T) * kTriF, 0.0f);
     P->tri_t_i.assign(static_cast<size_t>(T) * kTriI, -1);
+    int most_rows = 0;
+    P->row_map.assign(P->tile_start.size() * kGatherCols, 0xffffffffu);
     {
         constexpr int kRun = kTileTris / 4;  // tests per wave
         auto slot = [&](int p, int l) { return ldof[3 * static_cast<size_t>(p) + l]; };
@@ -534,13 +569,40 @@ std::string build_plan(int nv, int T, int n, int symmetry, const float *vtx, con
         };
         for (size_t tile = 0; tile < P->tile_start.size(); ++tile) {
             const int t0 = P->tile_start[tile], tc = P->tile_count[tile];
+            std::vector<char> taken(static_cast<size_t>(tc), 0);
+            auto open_edges = [&](int i) {  // edge neighbours not in a run yet
+                int c = 0;
+                for (int j = 0; j < tc; ++j)
+                    if (j != i && !taken[j] && n_shared(t0 + i, t0 + j) >= 2) ++c;
+                return c;
+            };
             for (int w0 = 0; w0 < tc; w0 += kRun) {
                 const int n = std::min(kRun, tc - w0), base = t0 + w0;
+                std::vector<int> run;
+                std::vector<char> in_run(kTileMaxDofs, 0);
+                while (static_cast<int>(run.size()) < n) {
+                    int best = -1, bf = 0, bo = 0;
+                    for (int i = 0; i < tc; ++i) {
+                        if (taken[i]) continue;
+                        int fresh = 0;
+                        for (int l = 0; l < 3; ++l) fresh += !in_run[slot(t0 + i, l)];
+                        if (best >= 0 && fresh > bf) continue;
+                        const int oe = open_edges(i);
+                        if (best < 0 || fresh < bf || oe < bo) {
+                            best = i;
+                            bf = fresh;
+                            bo = oe;
+                        }
+                    }
+                    taken[best] = 1;
+                    for (int l = 0; l < 3; ++l) in_run[slot(t0 + best, l)] = 1;
+                    run.push_back(t0 + best);
+                }
                 std::vector<char> used(static_cast<size_t>(n), 0);
                 auto free_edges = [&](int i) {
                     int c = 0;
                     for (int j = 0; j < n; ++j)
-                        if (j != i && !used[j] && n_shared(base + i, base + j) >= 2) ++c;
+                        if (j != i && !used[j] && n_shared(run[i], run[j]) >= 2) ++c;
                     return c;
                 };
                 std::vector<int> order;
@@ -553,7 +615,7 @@ std::string build_plan(int nv, int T, int n, int symmetry, const float *vtx, con
                     int best = -1, bs = -1, bf = 0;
                     for (int j = 0; j < n; ++j) {
                         if (used[j]) continue;
-                        const int sh = n_shared(base + cur, base + j), fe = free_edges(j);
+                        const int sh = n_shared(run[cur], run[j]), fe = free_edges(j);
                         if (sh > bs || (sh == bs && fe < bf)) {
                             best = j;
                             bs = sh;
@@ -564,7 +626,7 @@ std::string build_plan(int nv, int T, int n, int symmetry, const float *vtx, con
                 }
                 int held[3] = {-1, -1, -1};
                 for (int k = 0; k < n; ++k) {
-                    const int p = base + order[k];
+                    const int p = run[order[k]];
                     int o[3] = {-1, -1, -1};
                     bool placed[3] = {false, false, false};
                     for (int r = 0; r < 3; ++r)
@@ -591,7 +653,69 @@ std::string build_plan(int nv, int T, int n, int symmetry, const float *vtx, con
                     P->tri_t_i[q * kTriI + 23] = p;
                     for (int r = 0; r < 3; ++r) held[r] = slot(p, o[r]);
                 }
+                // Rows of the wave's table: the run's dofs numbered as they
+                // appear, a new segment where the table would overflow; the
+                // last test of a segment but the run's last carries its
+                // number of rows, row_map holds the last segment's.
+                std::vector<int> rows;
+                for (int k = 0; k < n; ++k) {
+                    int32_t *ti = &P->tri_t_i[static_cast<size_t>(base + k) * kTriI];
+                    int fresh = 0;
+                    for (int r = 0; r < 3; ++r)
+                        fresh += std::find(rows.begin(), rows.end(), ti[20 + r]) == rows.end();
+                    if (static_cast<int>(rows.size()) + fresh > P->run_rows) {
+                        P->tri_t_i[static_cast<size_t>(base + k - 1) * kTriI + 18] =
+                            static_cast<int32_t>(rows.size());
+                        rows.clear();
+                    }
+                    for (int r = 0; r < 3; ++r) {
+                        const auto it = std::find(rows.begin(), rows.end(), ti[20 + r]);
+                        const int at = static_cast<int>(it - rows.begin());
+                        if (it == rows.end()) rows.push_back(ti[20 + r]);
+                        ti[20 + r] = at;
+                    }
+                    most_rows = std::max(most_rows, static_cast<int>(rows.size()));
+                    ti[18] = 0;
+                }
+                for (size_t r = 0; r < rows.size(); ++r) {
+                    uint32_t &w = P->row_map[tile * kGatherCols + rows[r]];
+                    const int shift = 8 * (w0 / kRun);
+                    w = (w & ~(0xffu << shift)) | (static_cast<uint32_t>(r) << shift);
+                }
             }
+        }
+    }
+    P->run_rows = most_rows;
+    // Tile pairs with a touching combination: a shared vertex, or equal
+    // coordinate keys under an image mask.
+    {
+        const size_t nt = P->tile_start.size();
+        auto ids = [&](size_t tile, int word) {
+            std::vector<int32_t> v;
+            for (int i = 0; i < P->tile_count[tile]; ++i)
+                for (int l = 0; l < 3; ++l)
+                    v.push_back(P->tri_i_aos[static_cast<size_t>(P->tile_start[tile] + i) * kTriI + word + l]);
+            std::sort(v.begin(), v.end());
+            v.erase(std::unique(v.begin(), v.end()), v.end());
+            return v;
+        };
+        auto meet = [](const std::vector<int32_t> &a, const std::vector<int32_t> &b) {
+            size_t i = 0, j = 0;
+            while (i < a.size() && j < b.size()) {
+                if (a[i] == b[j]) return true;
+                if (a[i] < b[j]) ++i; else ++j;
+            }
+            return false;
+        };
+        std::vector<std::vector<std::vector<int32_t>>> key(nt);
+        for (size_t t = 0; t < nt; ++t)
+            for (int m = 0; m <= M; ++m) key[t].push_back(ids(t, 3 + 3 * m));
+        P->tile_touch.assign(P->tile_pairs.size() / 2, 0);
+        for (size_t tp = 0; tp < P->tile_touch.size(); ++tp) {
+            const auto &s = key[P->tile_pairs[2 * tp]], &t = key[P->tile_pairs[2 * tp + 1]];
+            bool touch = meet(t[0], s[0]);
+            for (int m = 1; m < M && !touch; ++m) touch = meet(t[1], s[1 + m]);
+            P->tile_touch[tp] = touch;
         }
     }
     P->tri_f_soa.assign(static_cast<size_t>(T) * kTriF, 0.0f);
