@@ -76,37 +76,6 @@ __device__ __forceinline__ float mask_sign(int mask, int bit) { return (mask & b
 
 constexpr double kInv2PiD = 0.15915494309189533577;
 
-// G and dG/dn_y at an observation point for d = y - x given in FP64: the
-// distance and the phase k r (in revolutions, reduced to [-1/2, 1/2]) are
-// formed in FP64, so a field point metres away keeps the phase accuracy of
-// the quadrature points; sin, cos and the amplitudes are FP32.
-__device__ __forceinline__ GD kernel_gd_far(double dx, double dy, double dz, float nx, float ny,
-                                            float nz, float k, double krev) {
-    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-    const bool ok = r2 > 1.0e-14;
-    const float r2f = ok ? (float)r2 : 1.0f;
-    const float rinv32 = __builtin_amdgcn_rsqf(r2f);
-    const float r32 = r2f * rinv32;
-    // one Newton step from the FP32 root: relative error ~1e-14
-    const double r = (double)r32 + fma(-(double)r32, (double)r32, r2) * (double)(0.5f * rinv32);
-    double t = r * krev;
-    t -= rint(t);
-    const float tf = (float)t;
-    const float s = __builtin_amdgcn_sinf(tf);
-    const float c = __builtin_amdgcn_cosf(tf);
-    const float rinv = ok ? rinv32 : 0.0f;
-    const float scale = kInv4Pi * rinv;
-    const float gre = c * scale, gim = s * scale;
-    const float proj = fmaf((float)dx, nx, fmaf((float)dy, ny, (float)dz * nz)) * rinv;
-    const float fre = -rinv;
-    GD o;
-    o.gre = gre;
-    o.gim = gim;
-    o.dre = (gre * fre - gim * k) * proj;
-    o.dim = (gre * k + gim * fre) * proj;
-    return o;
-}
-
 // ---------------------------------------------------------------------------
 // Regular pairs.
 // One block = one unordered pair {T, S} of tiles of up to 64 triangles, for
@@ -1259,6 +1228,11 @@ __global__ void k_robin_neumann(const int32_t *__restrict__ l2g, int T, int vpk,
 
 constexpr int kFieldChunk = 16;
 
+// Lanes own observation points.  Bound by the VALU: 29 FP32 operations, fract
+// and 4 transcendentals per evaluation.  The distance and phase of a triangle's
+// vertex 0 (per image) are formed in FP64; a point's distance differs from it
+// by (r^2 - R^2) / (r + R) in FP32, so the phase k r keeps FP64-grade accuracy
+// metres away without FP64 work per evaluation.
 template <int kMasks>
 __global__ __launch_bounds__(256) void k_field(DeviceGeometry g, const float *__restrict__ field_k,
                                                int vpk, const float *__restrict__ p,
@@ -1273,57 +1247,105 @@ __global__ __launch_bounds__(256) void k_field(DeviceGeometry g, const float *__
     const int b = blockIdx.z;  // vector; its wavenumber is field_k[b / vpk]
     const bool ok = o < n_obs;
     const int oo = ok ? o : 0;
-    const float ox = obs[oo], oy = obs[n_obs + oo], oz = obs[2 * n_obs + oo];
-    const float k = field_k[b / vpk];
+    // the observation point under every image (mirroring it instead of the
+    // source leaves the triangle's record as it is)
+    float om[kMasks][3];
+#pragma unroll
+    for (int m = 0; m < kMasks; ++m)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            om[m][c] = obs[(size_t)c * n_obs + oo] * mask_sign(g.masks[m], 1 << c);
+    const float k = in_vgpr(field_k[b / vpk]);
+    const float krev = in_vgpr(k * kInv2Pi);
+    const double krev64 = (double)k * kInv2PiD;
     const float *pb = p + (size_t)b * p_stride * 2;
     const float *qb = q + (size_t)b * T * 2;
     float acc_re = 0.f, acc_im = 0.f;
     const int t_begin = blockIdx.y * kFieldChunk;
     const int t_end = min(T, t_begin + kFieldChunk);
-    const double ox64 = ox, oy64 = oy, oz64 = oz;
-    const double krev64 = (double)k * kInv2PiD;
     for (int t = t_begin; t < t_end; ++t) {
-        const float *tf = g.tri_f_aos + (size_t)t * kTriF;
-        const int32_t *ti = g.tri_i_aos + (size_t)t * kTriI;
-        const float p0r = pb[2 * ti[0]], p0i = pb[2 * ti[0] + 1];
-        const float p1r = pb[2 * ti[1]], p1i = pb[2 * ti[1] + 1];
-        const float p2r = pb[2 * ti[2]], p2i = pb[2 * ti[2] + 1];
-        const float qre = qb[2 * ti[19]], qim = qb[2 * ti[19] + 1];
-        const float jac = tf[22];
-        // vertex 0 and the two edges in FP64 (the vertices are exact floats)
-        double v0[3], e1[3], e2[3];
+        // test-side records: points as offsets from vertex 0
+        const float *tf = g.tri_t_f + (size_t)t * kTriF;
+        const int32_t *ti = g.tri_t_i + (size_t)t * kTriI;
+        const float jac = tf[22] * kInv4Pi;
+        float pv[2][3], qv[2];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            v0[c] = tf[23 + c];
-            e1[c] = (double)tf[26 + c] - v0[c];
-            e2[c] = (double)tf[29 + c] - v0[c];
+        for (int c = 0; c < 2; ++c) {
+#pragma unroll
+            for (int l = 0; l < 3; ++l) pv[c][l] = pb[2 * ti[l] + c] * jac;
+            qv[c] = -qb[2 * ti[19] + c] * jac;
         }
-        float tre = 0.f, tim = 0.f;
+        float xo[18], pw[2][6], qw[2][6];
 #pragma unroll
-        for (int a = 0; a < 6; ++a) {
-            const float xi = (float)kRule6X[a], eta = (float)kRule6Y[a];
-            const float b0 = 1.0f - xi - eta;
-            const float pr = b0 * p0r + xi * p1r + eta * p2r;
-            const float pi = b0 * p0i + xi * p1i + eta * p2i;
-            const float w = (float)kRule6W[a];
-            double y[3];
+        for (int j = 0; j < 18; ++j) xo[j] = in_vgpr(tf[j]);
 #pragma unroll
-            for (int c = 0; c < 3; ++c) y[c] = fma(kRule6X[a], e1[c], fma(kRule6Y[a], e2[c], v0[c]));
+        for (int a = 0; a < 6; ++a)
 #pragma unroll
-            for (int m = 0; m < kMasks; ++m) {
-                const int mask = g.masks[m];
-                const float sx = mask_sign(mask, 1), sy = mask_sign(mask, 2), sz = mask_sign(mask, 4);
-                const GD v = kernel_gd_far(sx * y[0] - ox64, sy * y[1] - oy64, sz * y[2] - oz64,
-                                           sx * tf[18], sy * tf[19], sz * tf[20], k, krev64);
-                // (dG/dn p - G q) w
-                const float cre = (v.dre * pr - v.dim * pi) - (v.gre * qre - v.gim * qim);
-                const float cim = (v.dre * pi + v.dim * pr) - (v.gre * qim + v.gim * qre);
-                tre = fmaf(cre, w, tre);
-                tim = fmaf(cim, w, tim);
+            for (int c = 0; c < 2; ++c) {
+                pw[c][a] = fmaf((float)(kRule6W[a] * rule6_phi(a, 0)), pv[c][0],
+                                fmaf((float)(kRule6W[a] * rule6_phi(a, 1)), pv[c][1],
+                                     (float)(kRule6W[a] * rule6_phi(a, 2)) * pv[c][2]));
+                qw[c][a] = (float)kRule6W[kRule6Group[a]] * qv[c];
             }
+#pragma unroll
+        for (int m = 0; m < kMasks; ++m) {
+            float D[3], Dl[3];
+            double R2 = 0.0;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const double d = (double)tf[23 + c] - (double)om[m][c];
+                D[c] = (float)d;
+                Dl[c] = (float)(d - (double)D[c]);
+                R2 = fma(d, d, R2);
+            }
+            const float hR = __builtin_amdgcn_rsqf(fmaxf((float)R2, 1.0e-30f));
+            const float R32 = (float)R2 * hR;
+            const double R = (double)R32 + fma(-(double)R32, (double)R32, R2) * (double)(0.5f * hR);
+            double td = R * krev64;
+            td -= rint(td);
+            const float tR = (float)td, Rf = (float)R;
+            const float proj = fmaf(D[0], tf[18], fmaf(D[1], tf[19], D[2] * tf[20]));
+            float r2[6], sd[6], rinv[6], sn[6], cs[6];
+#pragma unroll
+            for (int a = 0; a < 6; ++a) {
+                const float dx = (D[0] + xo[3 * a]) + Dl[0];
+                const float dy = (D[1] + xo[3 * a + 1]) + Dl[1];
+                const float dz = (D[2] + xo[3 * a + 2]) + Dl[2];
+                r2[a] = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                // r^2 - R^2 = (d + D) . xo
+                sd[a] = fmaf(dx + D[0], xo[3 * a],
+                             fmaf(dy + D[1], xo[3 * a + 1], (dz + D[2]) * xo[3 * a + 2]));
+            }
+            trans_begin();
+#pragma unroll
+            for (int a = 0; a < 6; ++a) rinv[a] = __builtin_amdgcn_rsqf(fmaxf(r2[a], 1.0e-14f));
+#pragma unroll
+            for (int a = 0; a < 6; ++a)
+                sn[a] = __builtin_amdgcn_rcpf(fmaf(r2[a], rinv[a], Rf));
+#pragma unroll
+            for (int a = 0; a < 6; ++a)
+                sn[a] = __builtin_amdgcn_fractf(fmaf(sd[a] * sn[a], krev, tR));
+#pragma unroll
+            for (int a = 0; a < 6; ++a) {
+                cs[a] = __builtin_amdgcn_cosf(sn[a]);
+                sn[a] = __builtin_amdgcn_sinf(sn[a]);
+            }
+            trans_end();
+            float tre = 0.0f, tim = 0.0f;
+#pragma unroll
+            for (int a = 0; a < 6; ++a) {
+                // e^{ikr}/r ((ik - 1/r) p proj/r - q)
+                const float ri = r2[a] > 1.0e-14f ? rinv[a] : 0.0f;
+                const float pr = proj * ri;
+                const float ar = pw[0][a] * pr, ai = pw[1][a] * pr;
+                const float xr = fmaf(-ri, ar, fmaf(-k, ai, qw[0][a])) * ri;
+                const float xi = fmaf(-ri, ai, fmaf(k, ar, qw[1][a])) * ri;
+                tre = fmaf(cs[a], xr, fmaf(-sn[a], xi, tre));
+                tim = fmaf(cs[a], xi, fmaf(sn[a], xr, tim));
+            }
+            acc_re += tre;
+            acc_im += tim;
         }
-        acc_re = fmaf(tre, jac, acc_re);
-        acc_im = fmaf(tim, jac, acc_im);
     }
     if (ok) {
         atomicAdd(out + ((size_t)b * n_obs + o) * 2, acc_re);
