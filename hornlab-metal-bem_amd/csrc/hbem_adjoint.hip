@@ -99,27 +99,47 @@ __device__ __forceinline__ AdjK adj_kernel_far(double dx, double dy, double dz, 
     return o;
 }
 
-// adj_kernel with the distance and the phase k r formed in FP64 from the
-// components of d (which the regular adjoint forms without cancellation,
-// from vertex-anchored offsets): the phase error no longer grows with k r.
+// 1/r and the reduced phase (revolutions) of six distances given as r^2 in
+// FP64, then sin and cos: the transcendentals of six evaluations as one run at
+// raised wave priority; both zero (so G is) for r^2 <= 1e-14.  A transcendental takes both issue ports of a SIMD for
+// 8 cycles; interleaved with FP32 work it also keeps two waves from pairing
+// their operations.  kComplexK: damp = e^{-k_im r}.
 template <bool kComplexK>
-__device__ __forceinline__ AdjK adj_kernel_p(double dx, double dy, double dz, float k, double krev,
-                                             float kim) {
-    const double r2d = fma(dx, dx, fma(dy, dy, dz * dz));
-    const bool ok = r2d > 1.0e-14;
-    const float r2 = ok ? (float)r2d : 1.0e-14f;
-    const float rinv = __builtin_amdgcn_rsqf(r2);
-    const float r32 = r2 * rinv;
-    const double rd = (double)r32 + fma(-(double)r32, (double)r32, r2d) * (double)(0.5f * rinv);
-    double td = rd * krev;
-    td -= rint(td);
-    const float t = (float)td;
-    const float r = (float)rd;
-    const float s = __builtin_amdgcn_sinf(t);
-    const float c = __builtin_amdgcn_cosf(t);
+__device__ __forceinline__ void adj_phases(const double (&r2d)[6], double krev, float kim,
+                                           float (&rinv)[6], float (&sn)[6], float (&cs)[6],
+                                           float (&damp)[6]) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+        rinv[i] = __builtin_amdgcn_rsqf(r2d[i] > 1.0e-14 ? (float)r2d[i] : 1.0e-14f);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+        const float r32 = (r2d[i] > 1.0e-14 ? (float)r2d[i] : 1.0e-14f) * rinv[i];
+        const double rd =
+            (double)r32 + fma(-(double)r32, (double)r32, r2d[i]) * (double)(0.5f * rinv[i]);
+        double td = rd * krev;
+        td -= rint(td);
+        sn[i] = (float)td;
+        if (kComplexK) damp[i] = (float)rd;
+    }
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+        cs[i] = __builtin_amdgcn_cosf(sn[i]);
+        sn[i] = __builtin_amdgcn_sinf(sn[i]);
+        if (kComplexK) damp[i] = __expf(-kim * damp[i]);
+        if (!(r2d[i] > 1.0e-14)) sn[i] = cs[i] = 0.0f;
+    }
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// G, H and G Q / r^2 from the parts above.
+template <bool kComplexK>
+__device__ __forceinline__ AdjK adj_factors(float rinv, float s, float c, float damp,
+                                            float k, float kim) {
     float sc = kInv4Pi * rinv;
-    if (kComplexK) sc *= __expf(-kim * r);
-    sc = ok ? sc : 0.0f;
+    if (kComplexK) sc *= damp;
     AdjK o;
     o.gre = c * sc;
     o.gim = s * sc;
@@ -434,12 +454,6 @@ __global__ __launch_bounds__(256, 2) void k_adjoint_regular(
     const float nhx = tfs[(size_t)18 * T + sdd], nhy = tfs[(size_t)19 * T + sdd],
                 nhz = tfs[(size_t)20 * T + sdd];
     const float nx = nhx * js, ny = nhy * js, nz = nhz * js;
-    int skey[kMaxMasks][3];
-#pragma unroll
-    for (int m = 0; m < kMaxMasks; ++m)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            skey[m][j] = m < g.n_masks ? tis[(size_t)(6 + 3 * m + j) * T + sdd] : -2;
     const int s_orig = tis[(size_t)19 * T + sdd];
     const float *pb = p + (size_t)b * ld * 2;
     const float *lb = lam + (size_t)b * ld * 2;
@@ -466,22 +480,14 @@ __global__ __launch_bounds__(256, 2) void k_adjoint_regular(
 
     double dy[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, dn[3] = {0, 0, 0}, dnh = 0.0;
     double ds[2] = {0, 0};
-    const float *tfa = g.tri_f_aos;
-    const int32_t *tia = g.tri_i_aos;
+    // test-side records: points as offsets from vertex 0
+    const float *tfa = g.tri_t_f;
+    const int32_t *tia = g.tri_t_i;
     for (int t = t_begin; t < t_end; ++t) {
         const float *tf = tfa + (size_t)t * kTriF;
         const int32_t *ti = tia + (size_t)t * kTriI;
         const float jt = tf[22];
-        // test points as vertex 0 plus X_a e1 + Y_a e2, the offsets formed
-        // where they are used (registers: the kernel's occupancy is set by
-        // its VGPR count)
-        float v0t[3], te1[3], te2[3];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            v0t[c] = tf[23 + c];
-            te1[c] = tf[26 + c] - v0t[c];
-            te2[c] = tf[29 + c] - v0t[c];
-        }
+        const float *v0t = tf + 23;
         // L_a = rw w_a |N_t| sum_i conj(lambda_i) phi_i(a)
         float lr[3], li[3];
 #pragma unroll
@@ -504,9 +510,11 @@ __global__ __launch_bounds__(256, 2) void k_adjoint_regular(
         for (int m = 0; m < g.n_masks; ++m) {
             bool touch = false;
 #pragma unroll
-            for (int i = 0; i < 3; ++i)
+            for (int j = 0; j < 3; ++j) {
+                const int key = tis[(size_t)(6 + 3 * m + j) * T + sdd];
 #pragma unroll
-                for (int j = 0; j < 3; ++j) touch |= ti[6 + i] == skey[m][j];
+                for (int i = 0; i < 3; ++i) touch |= ti[6 + i] == key;
+            }
             if (touch || !live) continue;
             const int mask = g.masks[m];
             const float sx = msign(mask, 1), sy = msign(mask, 2), sz = msign(mask, 4);
@@ -515,19 +523,26 @@ __global__ __launch_bounds__(256, 2) void k_adjoint_regular(
                         az = v0s[2] - sz * v0t[2];
 #pragma unroll
             for (int a = 0; a < 6; ++a) {
-                const float xoa = fmaf((float)kRule6X[a], te1[0], (float)kRule6Y[a] * te2[0]);
-                const float yoa = fmaf((float)kRule6X[a], te1[1], (float)kRule6Y[a] * te2[1]);
-                const float zoa = fmaf((float)kRule6X[a], te1[2], (float)kRule6Y[a] * te2[2]);
-                const float bx = ax - sx * xoa, by = ay - sy * yoa, bz = az - sz * zoa;
+                const float bx = ax - sx * tf[3 * a], by = ay - sy * tf[3 * a + 1],
+                            bz = az - sz * tf[3 * a + 2];
                 const float alr = Lr[a] * qr - Li[a] * qi, ali = Lr[a] * qi + Li[a] * qr;
                 float gxa = 0.0f, gya = 0.0f, gza = 0.0f;
                 float gsr = 0.0f, gsi = 0.0f;  // sum_b w_b G
                 float ja = 0.0f;               // sum_b w_b (-Re[beta H] (r . N))
+                double r2d[6];
+                float rinv[6], sn[6], cs[6], damp[6];
+#pragma unroll
+                for (int bb = 0; bb < 6; ++bb) {
+                    const double rx = bx + ys[3 * bb], ry = by + ys[3 * bb + 1],
+                                 rz = bz + ys[3 * bb + 2];
+                    r2d[bb] = fma(rx, rx, fma(ry, ry, rz * rz));
+                }
+                adj_phases<kComplexK>(r2d, krev, kim, rinv, sn, cs, damp);
 #pragma unroll
                 for (int bb = 0; bb < 6; ++bb) {
                     const float wb = (float)kRule6W[bb];
                     const float rx = bx + ys[3 * bb], ry = by + ys[3 * bb + 1], rz = bz + ys[3 * bb + 2];
-                    const AdjK K = adj_kernel_p<kComplexK>(rx, ry, rz, k, krev, kim);
+                    const AdjK K = adj_factors<kComplexK>(rinv[bb], sn[bb], cs[bb], damp[bb], k, kim);
                     const float rn = fmaf(rx, nx, fmaf(ry, ny, rz * nz));
                     const float btr = (Lr[a] * Pr[bb] - Li[a] * Pi[bb]) * wb;
                     const float bti = (Lr[a] * Pi[bb] + Li[a] * Pr[bb]) * wb;
