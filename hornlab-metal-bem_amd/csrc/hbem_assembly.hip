@@ -443,6 +443,18 @@ __host__ __device__ constexpr int regular_wave_lds(int rows, int dofs) {
     return kStageBytes / 16 + rows * dofs;
 }
 
+// Sum over the wave (in every lane), in data-parallel moves within rows of 16
+// lanes and row broadcasts instead of LDS permutes.
+__device__ __forceinline__ float wave_sum(float x) {
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x111, 0xf, 0xf, true));
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x112, 0xf, 0xf, true));
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x114, 0xf, 0xf, true));
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x118, 0xf, 0xf, true));
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x142, 0xa, 0xf, false));
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x143, 0xc, 0xf, false));
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+}
+
 // One tile pair (pair index tp) at one frequency (b) of the regular
 // assembly: the block body shared by the single-mesh kernel and the
 // multi-mesh launch of a session group.
@@ -557,6 +569,28 @@ __device__ __forceinline__ void regular_tile_pair(
 #pragma unroll
             for (int r = 0; r < 3; ++r) dF[c][i][r] = dR[c][i][r] = 0.0f;
     int row_dof = -1;  // dof of table row `lane`
+    // the sum of the staged values of the lane's trial dof
+    auto gather = [&]() {
+        v4f sum = zero4;
+        auto add4 = [&](uint32_t w) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum += stage[(w >> (8 * e)) & 0xffu];
+        };
+        add4(list[0]);
+        if (groups > 1) add4(list[1]);
+        for (int e = kGatherHeld; e < groups; ++e) add4(opaque(g.gather)[list_at + e * kGatherCols]);
+        return sum;
+    };
+    // right-hand side of the first source: of the lane's trial dof, and of the
+    // test dof of table row `lane`
+    float col_rhs[2] = {0.0f, 0.0f}, row_rhs[2] = {0.0f, 0.0f};
+    float *rhs_b = rhs + (size_t)b * n_src * rhs_stride * 2;
+    auto add_rhs = [&](float *dst, int dof, float re, float im) {
+        if (re != 0.0f || im != 0.0f) {
+            atomicAdd(dst + (size_t)dof * 2, re);
+            atomicAdd(dst + (size_t)dof * 2 + 1, im);
+        }
+    };
     auto flush = [&](int r, int to_row, int dof) {
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
@@ -567,14 +601,7 @@ __device__ __forceinline__ void regular_tile_pair(
         if (lane == to_row) row_dof = dof;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        v4f sum = zero4;
-        auto add4 = [&](uint32_t w) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) sum += stage[(w >> (8 * e)) & 0xffu];
-        };
-        add4(list[0]);
-        if (groups > 1) add4(list[1]);
-        for (int e = kGatherHeld; e < groups; ++e) add4(opaque(g.gather)[list_at + e * kGatherCols]);
+        const v4f sum = gather();
         if (col_ok) table[to_row * snd + lane] += sum;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -610,6 +637,8 @@ __device__ __forceinline__ void regular_tile_pair(
                 table[r * snd + lane] = zero4;
             }
         }
+        if (lane < rows) add_rhs(opaque(rhs_b), row_dof, row_rhs[0], row_rhs[1]);
+        row_rhs[0] = row_rhs[1] = 0.0f;
     };
     int rec = 0;
     if (n_tests > 0)
@@ -705,39 +734,44 @@ __device__ __forceinline__ void regular_tile_pair(
         if (src) {
             const float gsc = gscale * cur.jac;  // sF / sR carry no Jacobian
             const float *q_s = opaque(q);
-            const int32_t *ids = opaque(g.tri_i_soa);
-            int sdof[3];
-#pragma unroll
-            for (int l = 0; l < 3; ++l) sdof[l] = ids[(size_t)l * T + tr];
             for (int sv = 0; sv < n_src; ++sv) {
-                float *rb = opaque(rhs) + ((size_t)b * n_src + sv) * rhs_stride * 2;
-                const size_t lq = (((size_t)b * n_src + sv) * T + orig) * 2;
-                const float qre = trial_ok ? q_s[lq] : 0.0f, qim = trial_ok ? q_s[lq + 1] : 0.0f;
+                float *rb = opaque(rhs_b) + (size_t)sv * rhs_stride * 2;
+                const size_t q0 = ((size_t)b * n_src + sv) * T;
+                const float qre = fwd ? q_s[(q0 + orig) * 2] : 0.0f;
+                const float qim = fwd ? q_s[(q0 + orig) * 2 + 1] : 0.0f;
                 if (__any(qre != 0.0f || qim != 0.0f)) {
-                    // rhs_t += 2^planes SLP(t, s) q_s, reduced over the wave
+                    // rhs_t += 2^planes SLP(t, s) q_s, summed over the wave
 #pragma unroll
                     for (int i = 0; i < 3; ++i) {
-                        float cre = fwd ? (sF[i][0] * qre - sF[i][1] * qim) * gsc : 0.0f;
-                        float cim = fwd ? (sF[i][0] * qim + sF[i][1] * qre) * gsc : 0.0f;
-#pragma unroll
-                        for (int off = 32; off >= 1; off >>= 1) {
-                            cre += __shfl_xor(cre, off);
-                            cim += __shfl_xor(cim, off);
-                        }
-                        if (lane == 0) {
-                            atomicAdd(rb + (size_t)cur.dof[i] * 2, cre);
-                            atomicAdd(rb + (size_t)cur.dof[i] * 2 + 1, cim);
+                        const float re = wave_sum((sF[i][0] * qre - sF[i][1] * qim) * gsc);
+                        const float im = wave_sum((sF[i][0] * qim + sF[i][1] * qre) * gsc);
+                        if (sv == 0) {
+                            row_rhs[0] += lane == cur.row[i] ? re : 0.0f;
+                            row_rhs[1] += lane == cur.row[i] ? im : 0.0f;
+                        } else if (lane == 0) {
+                            add_rhs(rb, cur.dof[i], re, im);
                         }
                     }
                 }
-                const size_t tq = (((size_t)b * n_src + sv) * T + torig) * 2;
-                const float tqre = q_s[tq], tqim = q_s[tq + 1];
-                if ((tqre != 0.0f || tqim != 0.0f) && rev) {
-                    // rhs_s += 2^planes SLP(s, t) q_t
+                const float tqre = q_s[(q0 + torig) * 2], tqim = q_s[(q0 + torig) * 2 + 1];
+                if (tqre != 0.0f || tqim != 0.0f) {
+                    // rhs_s += 2^planes SLP(s, t) q_t, gathered per trial dof
+                    const float gs = rev ? gsc : 0.0f;
 #pragma unroll
-                    for (int i = 0; i < 3; ++i) {
-                        atomicAdd(rb + (size_t)sdof[i] * 2, (sR[i][0] * tqre - sR[i][1] * tqim) * gsc);
-                        atomicAdd(rb + (size_t)sdof[i] * 2 + 1, (sR[i][0] * tqim + sR[i][1] * tqre) * gsc);
+                    for (int j = 0; j < 3; ++j)
+                        stage[64 * j + lane] = (v4f){(sR[j][0] * tqre - sR[j][1] * tqim) * gs,
+                                                     (sR[j][0] * tqim + sR[j][1] * tqre) * gs, 0.0f,
+                                                     0.0f};
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    const v4f sum = gather();
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    if (sv == 0) {
+                        col_rhs[0] += sum[0];
+                        col_rhs[1] += sum[1];
+                    } else if (col_ok) {
+                        add_rhs(rb, col_dof, sum[0], sum[1]);
                     }
                 }
             }
@@ -751,6 +785,8 @@ __device__ __forceinline__ void regular_tile_pair(
                 flush(r, cur.row[r], cur.dof[r]);
         if (cur.seg > 0) write_table(cur.seg);
     }
+    if (col_ok) add_rhs(rhs_b, col_dof, col_rhs[0], col_rhs[1]);
+    if (row_dof >= 0) add_rhs(rhs_b, row_dof, row_rhs[0], row_rhs[1]);
     __syncthreads();
     // The sum of the four tables to A, a wave's lanes on consecutive rows of one
     // column of A (its atomics share cache lines): for F lane = test dof and the
