@@ -868,10 +868,17 @@ __global__ __launch_bounds__(256, 2) void k_assemble_regular_multi(
 
 constexpr int kSgRun = 32;
 
-// Block (bx, by) of the singular-class assembly (4 waves of classes, kFB
-// frequencies): the body shared by the single-mesh kernel and the
-// multi-mesh launch.
-template <bool kComplexK, int kFB>
+// Block (bx, by) of the singular-class assembly, kFB frequencies: the body
+// shared by the single-mesh kernel and the multi-mesh launch.  kSplit = 1: four
+// waves of 64 classes.  kSplit > 1: one group of 64 classes, its runs of points
+// dealt to kSplit waves whose FP64 sums are added in LDS (small meshes and
+// sweeps, where whole rules per wave leave most of the chip idle).
+//
+// A wave keeps the points of its current run in LDS (the next run's loads are
+// in flight meanwhile) and reads them as broadcasts into vector registers: with
+// scalar operands the 48 block sums per point and frequency pair issue at half
+// rate.
+template <bool kComplexK, int kFB, int kSplit>
 __device__ __forceinline__ void singular_block(
     const DeviceGeometry &g, int bx, int by, const float *__restrict__ rule, int n_batch,
     const float *__restrict__ k_real, const float *__restrict__ k_imag,
@@ -879,7 +886,11 @@ __device__ __forceinline__ void singular_block(
     float *__restrict__ A, int64_t lda, int64_t a_stride, float *__restrict__ rhs,
     int64_t rhs_stride) {
     const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(bx * 4 + (threadIdx.x >> 6));
+    const int part = kSplit > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    // split groups start with the vertex pairs: the coincident ones carry the
+    // mass terms, the largest summands of their entries, which round least
+    // when they are added last
+    const int w = kSplit > 1 ? g.sg_waves[0] + g.sg_waves[1] + g.sg_waves[2] - 1 - bx : __builtin_amdgcn_readfirstlane(bx * 4 + (threadIdx.x >> 6));
     const int w1 = g.sg_waves[0], w2 = w1 + g.sg_waves[1], w3 = w2 + g.sg_waves[2];
     if (w >= w3) return;
     const int kind = w < w1 ? 0 : (w < w2 ? 1 : 2);
@@ -901,12 +912,17 @@ __device__ __forceinline__ void singular_block(
 #pragma unroll
     for (int f = 0; f < kFB; ++f) {
         const int b = min(b0 + f, n_batch - 1);
-        kk[f] = k_real[b];
-        krev[f] = kk[f] * kInv2Pi;
-        kim[f] = kComplexK ? k_imag[b] : 0.0f;
+        kk[f] = in_vgpr(k_real[b]);
+        krev[f] = in_vgpr(kk[f] * kInv2Pi);
+        kim[f] = kComplexK ? in_vgpr(k_imag[b]) : 0.0f;
     }
 
-    const float *__restrict__ rp = rule + (size_t)g.sg_rule_offset[kind] * kSgRule;
+    constexpr int kWaves = kSplit > 1 ? kSplit : 4;
+    static_assert(kSgRun * kSgRule == 4 * 128, "a run is two 16-byte words per lane");
+    __shared__ v4f rule_s[kWaves][128];
+    v4f *run_s = rule_s[threadIdx.x >> 6];
+    const v4f *__restrict__ rp =
+        reinterpret_cast<const v4f *>(rule + (size_t)g.sg_rule_offset[kind] * kSgRule) + lane;
     const int cnt = g.sg_rule_count[kind];
     double dd[kFB][9][2], ds[kFB][3][2];
 #pragma unroll
@@ -916,7 +932,19 @@ __device__ __forceinline__ void singular_block(
 #pragma unroll
         for (int i = 0; i < 3; ++i) ds[f][i][0] = ds[f][i][1] = 0.0;
     }
-    for (int p0 = 0; p0 < cnt; p0 += kSgRun) {
+    int p0 = part * kSgRun;
+    v4f next[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) next[h] = rp[(size_t)min(p0, cnt - kSgRun) * 4 + 64 * h];
+    for (; p0 < cnt; p0 += kSplit * kSgRun) {
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            run_s[64 * h + lane] = next[h];
+            next[h] = rp[(size_t)min(p0 + kSplit * kSgRun, cnt - kSgRun) * 4 + 64 * h];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         float ad[kFB][9][2], as[kFB][3][2];
 #pragma unroll
         for (int f = 0; f < kFB; ++f) {
@@ -925,72 +953,85 @@ __device__ __forceinline__ void singular_block(
 #pragma unroll
             for (int i = 0; i < 3; ++i) as[f][i][0] = as[f][i][1] = 0.0f;
         }
-        // Two-stage software pipeline over the points: the scalar loads of
-        // the next point are in flight while the current one is evaluated.
-        // distance vector of a point (its first use of the point's loads)
-        auto dist = [&](const float (&pt)[kSgRule], float &rx, float &ry, float &rz) {
-            const float dx = pt[0], dy = pt[1], xs = pt[2], ys = pt[3];
-            rx = fmaf(ys, g2x, fmaf(xs, g1x, fmaf(dy, e2x, fmaf(dx, e1x, r0x))));
-            ry = fmaf(ys, g2y, fmaf(xs, g1y, fmaf(dy, e2y, fmaf(dx, e1y, r0y))));
-            rz = fmaf(ys, g2z, fmaf(xs, g1z, fmaf(dy, e2z, fmaf(dx, e1z, r0z))));
+        // kP points per step, the next ones in flight; their transcendentals
+        // as one run at raised wave priority.
+        constexpr int kP = kFB > 1 ? 1 : 2;
+        auto load = [&](int p, v4f (&pt)[kP][4]) {
+#pragma unroll
+            for (int h = 0; h < kP; ++h)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) pt[h][j] = run_s[(p + h) * 4 + j];
         };
-        auto eval_point = [&](const float (&pt)[kSgRule], float rx, float ry, float rz) {
-            const float r2raw = fmaf(rx, rx, fmaf(ry, ry, rz * rz));
-            const bool ok = r2raw > 1.0e-14f;
-            const float r2 = ok ? r2raw : 1.0e-14f;
-            const float rinv = __builtin_amdgcn_rsqf(r2);
-            const float r = r2 * rinv;
-            const float gs = ok ? kInv4Pi * rinv : 0.0f;
-            const float proj = fmaf(rx, nx, fmaf(ry, ny, rz * nz)) * rinv;
+        auto eval = [&](const v4f (&pt)[kP][4]) {
+            float r2[kP], pn[kP], rinv[kP], r[kP], sn[kP][kFB], cs[kP][kFB], damp[kP][kFB];
+            bool ok[kP];
 #pragma unroll
-            for (int f = 0; f < kFB; ++f) {
-                float t = r * krev[f];
-                t = t - __builtin_rintf(t);
-                const float sn = __builtin_amdgcn_sinf(t);
-                const float cs = __builtin_amdgcn_cosf(t);
-                float sc = gs;
-                if (kComplexK) sc *= __expf(-kim[f] * r);
-                const float gre = cs * sc, gim = sn * sc;
-                const float fre = kComplexK ? (-rinv - kim[f]) : -rinv;
-                const float pre = gre * proj, pim = gim * proj;
-                const float dre = fmaf(pre, fre, -pim * kk[f]);
-                const float dim = fmaf(pre, kk[f], pim * fre);
+            for (int h = 0; h < kP; ++h) {
+                const float dx = pt[h][0][0], dy = pt[h][0][1], xs = pt[h][0][2], ys = pt[h][0][3];
+                const float rx = fmaf(ys, g2x, fmaf(xs, g1x, fmaf(dy, e2x, fmaf(dx, e1x, r0x))));
+                const float ry = fmaf(ys, g2y, fmaf(xs, g1y, fmaf(dy, e2y, fmaf(dx, e1y, r0y))));
+                const float rz = fmaf(ys, g2z, fmaf(xs, g1z, fmaf(dy, e2z, fmaf(dx, e1z, r0z))));
+                const float r2raw = fmaf(rx, rx, fmaf(ry, ry, rz * rz));
+                ok[h] = r2raw > 1.0e-14f;
+                r2[h] = ok[h] ? r2raw : 1.0e-14f;
+                pn[h] = fmaf(rx, nx, fmaf(ry, ny, rz * nz));
+            }
+            trans_begin();
 #pragma unroll
-                for (int i = 0; i < 9; ++i) {
-                    ad[f][i][0] = fmaf(dre, pt[4 + i], ad[f][i][0]);
-                    ad[f][i][1] = fmaf(dim, pt[4 + i], ad[f][i][1]);
+            for (int h = 0; h < kP; ++h) rinv[h] = __builtin_amdgcn_rsqf(r2[h]);
+#pragma unroll
+            for (int h = 0; h < kP; ++h) {
+                r[h] = r2[h] * rinv[h];
+#pragma unroll
+                for (int f = 0; f < kFB; ++f) {
+                    const float t = r[h] * krev[f];
+                    sn[h][f] = t - __builtin_rintf(t);
                 }
+            }
 #pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    as[f][i][0] = fmaf(gre, pt[13 + i], as[f][i][0]);
-                    as[f][i][1] = fmaf(gim, pt[13 + i], as[f][i][1]);
+            for (int h = 0; h < kP; ++h)
+#pragma unroll
+                for (int f = 0; f < kFB; ++f) {
+                    cs[h][f] = __builtin_amdgcn_cosf(sn[h][f]);
+                    sn[h][f] = __builtin_amdgcn_sinf(sn[h][f]);
+                    if (kComplexK) damp[h][f] = __expf(-kim[f] * r[h]);
+                }
+            trans_end();
+#pragma unroll
+            for (int h = 0; h < kP; ++h) {
+                const float gs = ok[h] ? kInv4Pi * rinv[h] : 0.0f;
+                const float proj = pn[h] * rinv[h];
+#pragma unroll
+                for (int f = 0; f < kFB; ++f) {
+                    const float sc = kComplexK ? gs * damp[h][f] : gs;
+                    const float gre = cs[h][f] * sc, gim = sn[h][f] * sc;
+                    const float fre = kComplexK ? (-rinv[h] - kim[f]) : -rinv[h];
+                    const float pre = gre * proj, pim = gim * proj;
+                    const float dre = fmaf(pre, fre, -pim * kk[f]);
+                    const float dim = fmaf(pre, kk[f], pim * fre);
+#pragma unroll
+                    for (int i = 0; i < 9; ++i) {
+                        const float wi = pt[h][1 + i / 4][i % 4];
+                        ad[f][i][0] = fmaf(dre, wi, ad[f][i][0]);
+                        ad[f][i][1] = fmaf(dim, wi, ad[f][i][1]);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) {
+                        const float wi = pt[h][1 + (9 + i) / 4][(9 + i) % 4];
+                        as[f][i][0] = fmaf(gre, wi, as[f][i][0]);
+                        as[f][i][1] = fmaf(gim, wi, as[f][i][1]);
+                    }
                 }
             }
         };
-        float pa[kSgRule], pb[kSgRule];
-#pragma unroll
-        for (int j = 0; j < kSgRule; ++j) pa[j] = rp[(size_t)p0 * kSgRule + j];
-        // Scalar loads return out of order, so a wait on one point's loads
-        // is a wait on all: each point's loads are consumed (dist) before
-        // the next point's loads are issued, and the scheduling barriers keep
-        // that order.
-        for (int p = p0; p < p0 + kSgRun; p += 2) {
-            float rx, ry, rz;
-            dist(pa, rx, ry, rz);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int j = 0; j < kSgRule; ++j) pb[j] = rp[(size_t)(p + 1) * kSgRule + j];
-            __builtin_amdgcn_sched_barrier(0);
-            eval_point(pa, rx, ry, rz);
-            __builtin_amdgcn_sched_barrier(0);
-            dist(pb, rx, ry, rz);
-            __builtin_amdgcn_sched_barrier(0);
-            const int pn = (p + 2 < cnt) ? p + 2 : p;
-#pragma unroll
-            for (int j = 0; j < kSgRule; ++j) pa[j] = rp[(size_t)pn * kSgRule + j];
-            __builtin_amdgcn_sched_barrier(0);
-            eval_point(pb, rx, ry, rz);
-            __builtin_amdgcn_sched_barrier(0);
+        v4f pa[kP][4], pb[kP][4];
+        load(0, pa);
+#pragma unroll 1
+        for (int p = 0; p < kSgRun; p += 2 * kP) {
+            load(p + kP, pb);
+            eval(pa);
+            if (p + 2 * kP < kSgRun) load(p + 2 * kP, pa);
+            eval(pb);
         }
 #pragma unroll
         for (int f = 0; f < kFB; ++f) {
@@ -1007,6 +1048,28 @@ __device__ __forceinline__ void singular_block(
         }
     }
 
+    if constexpr (kSplit > 1) {
+        extern __shared__ double singular_lds[];  // [kSplit - 1][kFB * 24][64]
+        constexpr int kSums = kFB * 24;
+        auto each = [&](auto &&op) {
+#pragma unroll
+            for (int f = 0; f < kFB; ++f) {
+#pragma unroll
+                for (int i = 0; i < 18; ++i) op(f * 24 + i, dd[f][i >> 1][i & 1]);
+#pragma unroll
+                for (int i = 0; i < 6; ++i) op(f * 24 + 18 + i, ds[f][i >> 1][i & 1]);
+            }
+        };
+        if (part > 0)
+            each([&](int i, double &v) {
+                singular_lds[((size_t)(part - 1) * kSums + i) * 64 + lane] = v;
+            });
+        __syncthreads();
+        if (part > 0) return;
+#pragma unroll 1
+        for (int o = 0; o < kSplit - 1; ++o)
+            each([&](int i, double &v) { v += singular_lds[((size_t)o * kSums + i) * 64 + lane]; });
+    }
     const int orig = g.sg_i[(size_t)6 * np + c];
     if (orig < 0) return;
     const int T = g.n_triangles;
@@ -1060,28 +1123,28 @@ __device__ __forceinline__ void singular_block(
     }
 }
 
-template <bool kComplexK, int kFB>
-__global__ __launch_bounds__(256) void k_assemble_singular(
+template <bool kComplexK, int kFB, int kSplit>
+__global__ __launch_bounds__(kSplit > 1 ? 64 * kSplit : 256, 2) void k_assemble_singular(
     DeviceGeometry g, const float *__restrict__ rule, int n_batch,
     const float *__restrict__ k_real, const float *__restrict__ k_imag,
     const float *__restrict__ q, int n_src, const float *__restrict__ beta,
     float *__restrict__ A, int64_t lda, int64_t a_stride, float *__restrict__ rhs,
     int64_t rhs_stride) {
-    singular_block<kComplexK, kFB>(g, blockIdx.x, blockIdx.y, rule, n_batch, k_real, k_imag, q,
-                                   n_src, beta, A, lda, a_stride, rhs, rhs_stride);
+    singular_block<kComplexK, kFB, kSplit>(g, blockIdx.x, blockIdx.y, rule, n_batch, k_real, k_imag,
+                                           q, n_src, beta, A, lda, a_stride, rhs, rhs_stride);
 }
 
 // Singular classes of every member of a session group in one launch: block
 // x = (member, frequency group, wave block) flattened.
 template <bool kComplexK, int kFB>
-__global__ __launch_bounds__(256) void k_assemble_singular_multi(
+__global__ __launch_bounds__(256, 2) void k_assemble_singular_multi(
     const AssemblyJob *__restrict__ jobs, int n_jobs) {
     const int j = job_of_block(jobs, n_jobs, blockIdx.x, true);
     const AssemblyJob &jb = jobs[j];
     const int local = blockIdx.x - jb.block_begin_sing;
     const int waves = jb.g.sg_waves[0] + jb.g.sg_waves[1] + jb.g.sg_waves[2];
     const int nbx = (waves + 3) / 4;
-    singular_block<kComplexK, kFB>(jb.g, local % nbx, local / nbx, jb.g.sg_rule, jb.n_batch,
+    singular_block<kComplexK, kFB, 1>(jb.g, local % nbx, local / nbx, jb.g.sg_rule, jb.n_batch,
                                    jb.k_real, jb.k_imag, jb.q, jb.n_src, jb.beta, jb.A, jb.lda,
                                    jb.a_stride, jb.rhs, jb.rhs_stride);
 }
@@ -1498,22 +1561,34 @@ void launch_assemble_regular(const DeviceGeometry &g, int n_batch, const float *
         by_masks(std::false_type{});
 }
 
+// Fewer wave-sized pieces than this (two per SIMD) do not fill the chip.
+constexpr int64_t kSingularSplitWaves = 2048;
+
 void launch_assemble_singular(const DeviceGeometry &g, int n_batch, const float *k_real,
                               const float *k_imag, const float *q, int n_src, const float *beta,
                               float *A, int64_t lda, int64_t a_stride, float *rhs,
                               int64_t rhs_stride, hipStream_t stream) {
     const int waves = g.sg_waves[0] + g.sg_waves[1] + g.sg_waves[2];
     if (waves == 0 || n_batch <= 0) return;
-    constexpr int kFB = 2;
-    dim3 grid((waves + 3) / 4, (n_batch + kFB - 1) / kFB);
+    auto go = [&](auto complex_k, auto fb_t, auto split_t) {
+        constexpr bool kC = decltype(complex_k)::value;
+        constexpr int kFB = decltype(fb_t)::value, kSplit = decltype(split_t)::value;
+        const dim3 grid(kSplit > 1 ? waves : (waves + 3) / 4, (n_batch + kFB - 1) / kFB);
+        const size_t shm = kSplit > 1 ? (size_t)(kSplit - 1) * kFB * 24 * 64 * sizeof(double) : 0;
+        hipLaunchKernelGGL((k_assemble_singular<kC, kFB, kSplit>), grid,
+                           dim3(kSplit > 1 ? 64 * kSplit : 256), shm, stream, g, g.sg_rule, n_batch,
+                           k_real, k_imag, q, n_src, beta, A, lda, a_stride, rhs, rhs_stride);
+    };
+    auto by_size = [&](auto complex_k) {
+        if ((int64_t)waves * ((n_batch + 1) / 2) < kSingularSplitWaves)
+            go(complex_k, std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{});
+        else
+            go(complex_k, std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{});
+    };
     if (k_imag != nullptr)
-        hipLaunchKernelGGL((k_assemble_singular<true, kFB>), grid, dim3(256), 0, stream, g,
-                           g.sg_rule, n_batch, k_real, k_imag, q, n_src, beta, A, lda, a_stride, rhs,
-                           rhs_stride);
+        by_size(std::true_type{});
     else
-        hipLaunchKernelGGL((k_assemble_singular<false, kFB>), grid, dim3(256), 0, stream, g,
-                           g.sg_rule, n_batch, k_real, k_imag, q, n_src, beta, A, lda, a_stride, rhs,
-                           rhs_stride);
+        by_size(std::false_type{});
 }
 
 void launch_assemble_multi(const AssemblyJob *jobs_dev, const std::vector<AssemblyJob> &jobs,
