@@ -1,0 +1,148 @@
+"""Assembly and field kernels at the edges of their tiles, lists and splits,
+against the FP64 oracle.
+
+Matrix and right-hand side: an entry is a sum of a few dozen FP32 roundings of
+6e-8 of its largest partial sum, so 2e-6 relative bounds the whole.  Field: 6 T
+images terms summed in chunks of 16 triangles, the same bound.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle as O
+from meshes import buffers_from_arrays, horn_buffers, mesh_buffers, rel_l2, sphere_buffers
+
+pytestmark = pytest.mark.gpu
+
+
+def _session(buffers, plane=None):
+    from hornlab_metal_bem.native import HipBemSession
+
+    return HipBemSession.create_session(buffers, symmetry_plane=plane, check_open_edges=False)
+
+
+def _soup(n_tri, seed=0):
+    """Separate triangles with dofs of their own: three rows per test, so a
+    wave's table overflows within its run."""
+    rng = np.random.default_rng(seed)
+    c = rng.uniform(0.02, 0.3, (n_tri, 1, 3))
+    V = (c + rng.uniform(-0.01, 0.01, (n_tri, 3, 3))).reshape(-1, 3)
+    V[0, :2] = 0.0  # one vertex on the symmetry planes
+    E = np.arange(3 * n_tri).reshape(-1, 3)
+    return buffers_from_arrays(V.T, E.T, E, 3 * n_tri, np.full(n_tri, 2))
+
+
+def _fan(valence):
+    """Double cone: two vertices shared by ``valence`` triangles each, longer
+    than the list words a lane holds."""
+    a = 2 * np.pi * np.arange(valence) / valence
+    V = np.concatenate([np.stack([0.1 * np.cos(a), 0.1 * np.sin(a), 0 * a], 1),
+                        [[0, 0, 0.08], [0, 0, -0.05]]])
+    i = np.arange(valence)
+    j = (i + 1) % valence
+    F = np.concatenate([np.stack([i, j, np.full(valence, valence)], 1),
+                        np.stack([j, i, np.full(valence, valence + 1)], 1)])
+    return mesh_buffers(V, F.astype(np.int32), np.full(2 * valence, 2, np.int32))
+
+
+def _check_assembly(b, plane, k, kim=0.0, beta=None):
+    rng = np.random.default_rng(1)
+    T = b.n_triangles
+    q = (rng.standard_normal(T) + 1j * rng.standard_normal(T)).astype(np.complex64)
+    walls = {2: beta} if beta is not None else None
+    with _session(b, plane) as s:
+        A, rhs = s.assemble_standard_neumann(0.0, k, q, k_imag=kim, impedance_sources=walls)
+    rows = None if beta is None else np.where(b.physical_tags_i32 == 2, np.complex64(beta), 0)
+    Ao, ro, _ = O.assemble(O.Geometry.from_buffers(b, plane), float(np.float32(k)), q,
+                           kim=float(np.float32(kim)), beta=rows)
+    assert rel_l2(A, Ao) < 2e-6
+    assert rel_l2(rhs, ro) < 2e-6
+
+
+@pytest.mark.parametrize("n_tri", [1, 15, 16, 17, 18, 19, 37, 64, 65])
+def test_tables_that_overflow(require_gpu, n_tri):
+    _check_assembly(_soup(n_tri), None, 20.0)
+
+
+@pytest.mark.parametrize("plane", ["xz", "yz+xz"])
+def test_tables_that_overflow_with_images(require_gpu, plane):
+    _check_assembly(_soup(30), plane, 20.0, 0.3, 0.2 + 0.1j)
+
+
+@pytest.mark.parametrize("valence", [8, 9, 12, 13, 40])
+def test_long_column_lists(require_gpu, valence):
+    _check_assembly(_fan(valence), None, 30.0)
+
+
+@pytest.mark.parametrize("edge,plane", [(0.05, "yz+xz"), (0.03, "yz+xz"), (0.02, "yz+xz")])
+def test_quarter_horn_all_sources_and_walls(require_gpu, edge, plane):
+    _check_assembly(horn_buffers(edge_length=edge), plane, 60.0)
+    _check_assembly(horn_buffers(edge_length=edge), plane, 60.0, 0.5, 0.3 - 0.2j)
+
+
+@pytest.mark.parametrize("n_sources", [1, 2, 3])
+def test_sources_on_every_triangle(require_gpu, n_sources):
+    """Each source's right-hand side solves to the same pressure as alone."""
+    b = sphere_buffers(subdivisions=2)
+    rng = np.random.default_rng(2)
+    T, k = b.n_triangles, np.array([8.0], np.float32)
+    q = (rng.standard_normal((n_sources, 1, T)) + 1j * rng.standard_normal((n_sources, 1, T))).astype(np.complex64)
+    obs = np.array([[0.0], [0.0], [2.0]], np.float32)
+    with _session(b) as s:
+        r = s.assemble_solve_evaluate_standard_neumann_batch(
+            np.array([400.0]), k, q[0], obs, extra_neumann_dp0=q[1:] if n_sources > 1 else None)[0]
+    g = O.Geometry.from_buffers(b)
+    for i, got in enumerate([r, *r.extra_sources]):
+        A, rhs, _ = O.assemble(g, 8.0, q[i, 0])
+        assert rel_l2(got.pressure, O.solve(A, rhs)) < 2e-5  # cond(A) ~ 10
+
+
+def test_split_and_whole_singular_rules_agree(require_gpu):
+    """One frequency per call deals the singular rules over eight waves, 18 in
+    one call do not; the pressures differ by FP32 rounding times cond."""
+    b = sphere_buffers(subdivisions=3)
+    f = np.geomspace(100.0, 1200.0, 18)
+    k = (2 * np.pi * f / 343.0).astype(np.float32)
+    q = np.ones((18, b.n_triangles), np.complex64)
+    obs = np.array([[0.0], [0.0], [2.0]], np.float32)
+    with _session(b) as s:
+        whole = s.assemble_solve_evaluate_standard_neumann_batch(f, k, q, obs)
+        for i in (0, 9, 17):
+            one = s.assemble_solve_evaluate_standard_neumann_batch(f[i:i + 1], k[i:i + 1], q[i:i + 1], obs)
+            assert rel_l2(one[0].pressure, whole[i].pressure) < 2e-5
+
+
+@pytest.mark.parametrize("plane", [None, "yz+xz"])
+@pytest.mark.parametrize("n_obs", [1, 63, 64, 65, 257])
+def test_field_points_near_and_far(require_gpu, plane, n_obs):
+    """Points from 1 mm off the surface to 60 m away, k r up to 1.3e3."""
+    b = horn_buffers(edge_length=0.03, quarter=plane is not None)
+    rng = np.random.default_rng(3)
+    d = rng.standard_normal((3, n_obs))
+    obs = (d / np.linalg.norm(d, axis=0) * np.geomspace(0.3, 60.0, n_obs)).astype(np.float32)
+    tri = b.triangles_3xm_i32[:, rng.integers(0, b.n_triangles, n_obs)]
+    near = b.vertices_3xn_f32[:, tri].mean(axis=1) * np.float32(1.01) + np.float32(1e-3)
+    obs[:, ::4] = near[:, ::4]
+    k = np.array([20.0], np.float32)
+    p = (rng.standard_normal(b.p1_dof_count) + 1j * rng.standard_normal(b.p1_dof_count)).astype(np.complex64)
+    q = (20 * rng.standard_normal(b.n_triangles)).astype(np.complex64)
+    with _session(b, plane) as s:
+        got = s.evaluate_standard_exterior_batch(np.array([1000.0]), k, p[None], q[None], obs)[0]
+    want = O.field(O.Geometry.from_buffers(b, plane), 20.0, p, q, obs)
+    # near points: each term |p| jac w / (4 pi r^2) + |q| jac w / (4 pi r) of
+    # the sum carries about ten roundings of 6e-8 (its distance, formed from a
+    # vertex and an offset up to 30 times as long, more than its product), so
+    # 4e-6 of the terms' sum bounds the error (the identity image's terms; the
+    # others are farther)
+    X, Y, W = O.rule6()
+    v = b.vertices_3xn_f32[:, b.triangles_3xm_i32].astype(float)  # (3, 3, T)
+    y = np.einsum("bl,clt->cbt", np.stack([1 - X - Y, X, Y], 1), v)
+    r = np.linalg.norm(y[:, :, :, None] - obs[:, None, None, ::4], axis=0)
+    w = W[:, None, None] * (2 * b.triangle_areas_f32)[None, :, None] / (4 * np.pi)
+    terms = (w * (np.abs(p).max() / r ** 2 + np.abs(q)[None, :, None] / r)).sum((0, 1))
+    assert np.all(np.abs(got - want)[::4] < 4e-6 * terms)
+    far = np.ones(n_obs, bool)
+    far[::4] = False
+    if far.any():
+        assert rel_l2(got[far], want[far]) < 5e-6
