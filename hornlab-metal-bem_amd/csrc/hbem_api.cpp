@@ -908,7 +908,7 @@ void chief_solve(hbem_session *s, const hbem::LuWorkspace &w, int B, int S, int 
     s->chief_z64.reserve(sizeof(double) * ze.size());
     s->chief_r.reserve(sizeof(double) * ze.size());
     s->norms.reserve(sizeof(double) * 2 * std::max(BM, V));
-    hbem::lu_solve(w, s->chief_z.as<float>(), N, 2, st, m);
+    hbem::lu_solve(w, s->chief_z.as<float>(), N, 2, st, m, s->trsv_on ? &s->trsv[0] : nullptr);
     hbem::launch_fill_zero_f64(s->chief_z64.as<double>(), ze.size(), st);
     hbem::launch_axpy_f32_to_f64(s->chief_z.as<float>(), s->chief_z64.as<double>(), N, N, n, BM,
                                  nullptr, st);
@@ -919,7 +919,8 @@ void chief_solve(hbem_session *s, const hbem::LuWorkspace &w, int B, int S, int 
         hbem::launch_fill_zero(s->chief_z.as<float>(), zr.size(), st);
         hbem::launch_copy_f64_to_f32(s->chief_r.as<double>(), s->chief_z.as<float>(), N, N, n, BM,
                                      st);
-        hbem::lu_solve(w, s->chief_z.as<float>(), N, 2, st, m);
+        hbem::lu_solve(w, s->chief_z.as<float>(), N, 2, st, m,
+                       s->trsv_on ? &s->trsv[0] : nullptr);
         hbem::launch_axpy_f32_to_f64(s->chief_z.as<float>(), s->chief_z64.as<double>(), N, N, n,
                                      BM, nullptr, st);
     }
@@ -1070,7 +1071,7 @@ void solve_resident(hbem_session *s, int B, int S, int n, int N, const hbem_solv
         w.perm = s->lu_perm.as<int32_t>();
         w.pi = s->lu_pi.as<int32_t>();
         w.dinv = s->lu_dinv.as<float>();
-        s->trsv[0] = trsv_sync(s, 0, V, N, st);
+        s->trsv[0] = trsv_sync(s, 0, std::max(V, B * std::max(0, (int)opt.n_chief)), N, st);
         s->trsv[1] = trsv_sync(s, 1, B, N, st);
     }
     // The rcond iteration needs only the LU factors: it runs on the aux
@@ -1681,7 +1682,16 @@ int32_t hbem_adjoint_backward(hbem_session *s, const float *grad_field, double *
         hbem::LuWorkspace w{s->A.as<float>(), lda, a_stride, N, n, B, s->ipiv.as<int32_t>(),
                             s->info.as<int32_t>(), s->gl.as<int32_t>(), s->lu_scr_i.as<int32_t>(),
                             s->lu_scr_f.as<float>()};
-        hbem::lu_solve(w, s->adj_l32.as<float>(), N, 2, st);
+        // the forward's multi-workgroup solve context (one vector per system)
+        const hbem::TrsvSync *sync = nullptr;
+        if (s->trsv_on) {
+            w.lf = s->lu_lf.as<float>();
+            w.perm = s->lu_perm.as<int32_t>();
+            w.pi = s->lu_pi.as<int32_t>();
+            w.dinv = s->lu_dinv.as<float>();
+            sync = &s->trsv[0];
+        }
+        hbem::lu_solve(w, s->adj_l32.as<float>(), N, 2, st, 1, sync);
         hbem::launch_fill_zero_f64(s->adj_l64.as<double>(), (size_t)2 * B * N, st);
         hbem::launch_axpy_f32_to_f64(s->adj_l32.as<float>(), s->adj_l64.as<double>(), N, N, n, B,
                                      nullptr, st);
@@ -1692,7 +1702,7 @@ int32_t hbem_adjoint_backward(hbem_session *s, const float *grad_field, double *
             hbem::launch_fill_zero(s->adj_l32.as<float>(), (size_t)2 * B * N, st);
             hbem::launch_copy_f64_to_f32(s->adj_r64.as<double>(), s->adj_l32.as<float>(), N, N, n,
                                          B, st);
-            hbem::lu_solve(w, s->adj_l32.as<float>(), N, 2, st);
+            hbem::lu_solve(w, s->adj_l32.as<float>(), N, 2, st, 1, sync);
             hbem::launch_axpy_f32_to_f64(s->adj_l32.as<float>(), s->adj_l64.as<double>(), N, N, n,
                                          B, nullptr, st);
         }
