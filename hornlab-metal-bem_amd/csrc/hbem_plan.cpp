@@ -13,13 +13,16 @@
 #include <array>
 #include <cmath>
 #include <cstring>
+#include <future>
 #include <unordered_map>
-#include <unordered_set>
 
 #include "hbem_internal.h"
 
 namespace hbem {
 namespace {
+
+// Tasks on threads of their own where one can be started, else run by get().
+constexpr std::launch kAnyLaunch = std::launch::async | std::launch::deferred;
 
 struct Key {
     int64_t x, y, z;
@@ -190,6 +193,30 @@ SideMap side_map(int nv, int T, const float *vtx, const int32_t *tri, int t, int
     return m;
 }
 
+// Number of distinct (row dof, column dof) entries the pairs touch.  The pairs
+// come grouped by trial triangle; per column dof the rows are stamped.
+int64_t count_slots(int T, int n, const int32_t *l2g, const std::vector<PairRec> &pairs) {
+    std::vector<size_t> begin(static_cast<size_t>(T) + 1, 0);
+    for (const PairRec &p : pairs) begin[static_cast<size_t>(p.trial) + 1]++;
+    for (int t = 0; t < T; ++t) begin[t + 1] += begin[t];
+    std::vector<int32_t> start(static_cast<size_t>(n) + 1, 0), list(3 * static_cast<size_t>(T));
+    for (int i = 0; i < 3 * T; ++i) start[l2g[i] + 1]++;
+    for (int d = 0; d < n; ++d) start[d + 1] += start[d];
+    std::vector<int32_t> at(start.begin(), start.end() - 1), stamp(n, -1);
+    for (int t = 0; t < T; ++t)
+        for (int l = 0; l < 3; ++l) list[at[l2g[3 * t + l]]++] = t;
+    int64_t count = 0;
+    for (int col = 0; col < n; ++col)
+        for (int q = start[col]; q < start[col + 1]; ++q)
+            for (size_t i = begin[list[q]]; i < begin[list[q] + 1]; ++i)
+                for (int l = 0; l < 3; ++l) {
+                    int32_t &seen = stamp[l2g[3 * pairs[i].test + l]];
+                    count += seen != col;
+                    seen = col;
+                }
+    return count;
+}
+
 // Groups the full singular pair list into classes (see Plan::sg_f) and
 // writes the per-class records and the per-point rule tables.
 void build_singular_classes(int nv, int T, const float *vtx, const int32_t *tri,
@@ -205,8 +232,13 @@ void build_singular_classes(int nv, int T, const float *vtx, const int32_t *tri,
     // set maps onto itself); the coincident and edge rules do not, so their
     // classes keep one representative per parity.  Triangle indices fit 24
     // bits (build_plan rejects larger meshes).
-    std::unordered_map<uint64_t, int> index;
-    index.reserve(pairs.size());
+    // The pairs come grouped by trial triangle, so a table of one trial's
+    // classes is enough (open addressing, emptied by a new stamp).
+    struct Entry {
+        uint64_t key;
+        int stamp, cls;
+    };
+    std::vector<Entry> table(256, Entry{0, -1, 0});
     std::vector<Cls> cls[3];
     for (size_t i = 0; i < pairs.size(); ++i) {
         const PairRec &p = pairs[i];
@@ -217,13 +249,23 @@ void build_singular_classes(int nv, int T, const float *vtx, const int32_t *tri,
             key |= (par << 8) | (static_cast<uint64_t>(p.tl1) << 6) | (static_cast<uint64_t>(p.tl2) << 4) |
                    (static_cast<uint64_t>(p.sl1) << 2) | static_cast<uint64_t>(p.sl2);
         }
-        const uint64_t full = key;
-        auto it = index.find(full);
-        if (it == index.end()) {
-            index.emplace(full, static_cast<int>(cls[p.kind - 1].size()));
-            cls[p.kind - 1].push_back(Cls{static_cast<int>(i), 1});
-        } else {
-            cls[p.kind - 1][it->second].weight++;
+        if (i == 0 || p.trial != pairs[i - 1].trial) {
+            size_t end = i;
+            while (end < pairs.size() && pairs[end].trial == p.trial) ++end;
+            while (table.size() < 2 * (end - i)) table.assign(2 * table.size(), Entry{0, -1, 0});
+        }
+        size_t h = (key * 0x9e3779b97f4a7c15ull) >> 32;
+        for (;; ++h) {
+            Entry &e = table[h & (table.size() - 1)];
+            if (e.stamp != p.trial) {
+                e = Entry{key, p.trial, static_cast<int>(cls[p.kind - 1].size())};
+                cls[p.kind - 1].push_back(Cls{static_cast<int>(i), 1});
+                break;
+            }
+            if (e.key == key) {
+                cls[p.kind - 1][e.cls].weight++;
+                break;
+            }
         }
     }
     int np = 0;
@@ -239,9 +281,11 @@ void build_singular_classes(int nv, int T, const float *vtx, const int32_t *tri,
     P->sg_i.assign(static_cast<size_t>(kSgI) * np, 0);
     P->sg_adj.assign(static_cast<size_t>(kSgAdj) * np, 0);
     for (int p = 0; p < np; ++p) P->sg_i[static_cast<size_t>(6) * np + p] = -1;
-    int base = 0;
-    for (int k = 0; k < 3; ++k) {
-        for (size_t c = 0; c < cls[k].size(); ++c) {
+    // Records of classes [c0, c1) of kind k.
+    auto fill = [&](int k, size_t c0, size_t c1) {
+        int base = 0;
+        for (int j = 0; j < k; ++j) base += 64 * P->sg_waves[j];
+        for (size_t c = c0; c < c1; ++c) {
             const PairRec &pr = pairs[cls[k][c].rep];
             const int slot = base + static_cast<int>(c);
             const SideMap tmap = side_map(nv, T, vtx, tri, pr.test, pr.tm, pr.kind, pr.tl1, pr.tl2);
@@ -275,7 +319,15 @@ void build_singular_classes(int nv, int T, const float *vtx, const int32_t *tri,
             aj[static_cast<size_t>(6) * np + slot] = pr.tm | (pr.sm << 4);
             aj[static_cast<size_t>(7) * np + slot] = pr.test;
         }
-        base += 64 * P->sg_waves[k];
+    };
+    {
+        constexpr size_t kPart = 8192;  // classes per task
+        std::vector<std::future<void>> tasks;
+        for (int k = 0; k < 3; ++k)
+            for (size_t c = 0; c < cls[k].size(); c += kPart)
+                tasks.push_back(std::async(kAnyLaunch, fill, k, c,
+                                           std::min(cls[k].size(), c + kPart)));
+        for (auto &t : tasks) t.get();
     }
 
     P->sg_rule.clear();
@@ -385,6 +437,109 @@ std::string build_plan(int nv, int T, int n, int symmetry, const float *vtx, con
         kid[i] = static_cast<int32_t>(std::lower_bound(uniq.begin(), uniq.end(), keys[i]) -
                                       uniq.begin());
     auto key_id = [&](int m, int v) { return kid[static_cast<size_t>(m) * nv + v]; };
+
+    // Singular pair list and classes, beside the tiles and records below (they
+    // share only their inputs); an exception there comes back through get().
+    auto singular = std::async(kAnyLaunch, [&]() {
+        std::vector<PairRec> pairs;
+        pairs.reserve(static_cast<size_t>(T) * 16 * M);
+        auto append = [&](int test, int trial, int tm, int sm, Shared s) {
+            int kind;
+            if (s.count == 3) {
+                kind = 1;
+                s.tl1 = 0; s.tl2 = 1; s.sl1 = 0; s.sl2 = 1;
+            } else if (s.count == 2) {
+                kind = 2;
+            } else if (s.count == 1) {
+                kind = 3;
+            } else {
+                return;
+            }
+            pairs.push_back(PairRec{test, trial, tm, sm, kind, s.tl1, s.tl2, s.sl1, s.sl2});
+        };
+        auto shared_by_index = [&](int test, int trial) {
+            Shared s;
+            for (int i = 0; i < 3; ++i)
+                for (int j = 0; j < 3; ++j)
+                    if (tri[i * T + test] == tri[j * T + trial]) s.add(i, j);
+            return s;
+        };
+        auto shared_by_key = [&](int test, int trial, int tmi, int smi) {
+            Shared s;
+            const int tm = P->masks[tmi], sm = P->masks[smi];
+            for (int tfl = 0; tfl < 3; ++tfl) {
+                const int tk = key_id(tmi, tri[image_local(tfl, tm) * T + test]);
+                for (int sfl = 0; sfl < 3; ++sfl)
+                    if (tk == key_id(smi, tri[image_local(sfl, sm) * T + trial])) s.add(tfl, sfl);
+            }
+            return s;
+        };
+        // Incidence: id -> triangles (CSR), per mask.
+        const int nid = (symmetry == 0) ? nv : static_cast<int>(uniq.size());
+        std::vector<std::vector<int32_t>> start(M), list(M);
+        for (int m = 0; m < (symmetry == 0 ? 1 : M); ++m) {
+            start[m].assign(static_cast<size_t>(nid) + 1, 0);
+            list[m].resize(static_cast<size_t>(T) * 3);
+            auto idof = [&](int t, int l) {
+                const int v = tri[l * T + t];
+                return symmetry == 0 ? v : key_id(m, v);
+            };
+            for (int t = 0; t < T; ++t)
+                for (int l = 0; l < 3; ++l) start[m][idof(t, l) + 1]++;
+            for (int i = 0; i < nid; ++i) start[m][i + 1] += start[m][i];
+            std::vector<int32_t> cur(start[m].begin(), start[m].end() - 1);
+            for (int t = 0; t < T; ++t)
+                for (int l = 0; l < 3; ++l) list[m][cur[idof(t, l)]++] = t;
+        }
+        std::vector<int32_t> stamp(T, 0), cand;
+        int st = 0;
+        for (int trial = 0; trial < T; ++trial) {
+            if (symmetry == 0) {
+                ++st;
+                cand.clear();
+                for (int l = 0; l < 3; ++l) {
+                    const int v = tri[l * T + trial];
+                    for (int p = start[0][v]; p < start[0][v + 1]; ++p) {
+                        const int test = list[0][p];
+                        if (stamp[test] != st) {
+                            stamp[test] = st;
+                            cand.push_back(test);
+                        }
+                    }
+                }
+                for (int test : cand) append(test, trial, 0, 0, shared_by_index(test, trial));
+                continue;
+            }
+            for (int smi = 0; smi < M; ++smi)
+                for (int tmi = 0; tmi < M; ++tmi) {
+                    ++st;
+                    cand.clear();
+                    for (int l = 0; l < 3; ++l) {
+                        const int id = key_id(smi, tri[l * T + trial]);
+                        for (int p = start[tmi][id]; p < start[tmi][id + 1]; ++p) {
+                            const int test = list[tmi][p];
+                            if (stamp[test] != st) {
+                                stamp[test] = st;
+                                cand.push_back(test);
+                            }
+                        }
+                    }
+                    for (int test : cand) {
+                        const Shared s = (tmi == 0 && smi == 0) ? shared_by_index(test, trial)
+                                                                : shared_by_key(test, trial, tmi, smi);
+                        append(test, trial, P->masks[tmi], P->masks[smi], s);
+                    }
+                }
+        }
+        P->kind_count[0] = P->kind_count[1] = P->kind_count[2] = 0;
+        P->image_pairs = 0;
+        for (const PairRec &pr : pairs) {
+            P->kind_count[pr.kind - 1]++;
+            if (pr.tm != 0 || pr.sm != 0) P->image_pairs++;
+        }
+        P->unique_slots = count_slots(T, n, l2g, pairs);
+        build_singular_classes(nv, T, vtx, tri, l2g, areas, normals, pairs, P);
+    });
 
     // Device triangle order: Morton order of the centroids, so that runs of
     // consecutive triangles (tiles) cover compact patches with few distinct
@@ -561,61 +716,53 @@ std::string build_plan(int nv, int T, int n, int symmetry, const float *vtx, con
     {
         constexpr int kRun = kTileTris / 4;  // tests per wave
         auto slot = [&](int p, int l) { return ldof[3 * static_cast<size_t>(p) + l]; };
-        auto n_shared = [&](int p, int q) {
-            int c = 0;
-            for (int a = 0; a < 3; ++a)
-                for (int b = 0; b < 3; ++b) c += slot(p, a) == slot(q, b);
-            return c;
-        };
+        static_assert(kTileTris <= 64 && kTileMaxDofs <= 64, "one word per set");
         for (size_t tile = 0; tile < P->tile_start.size(); ++tile) {
             const int t0 = P->tile_start[tile], tc = P->tile_count[tile];
-            std::vector<char> taken(static_cast<size_t>(tc), 0);
-            auto open_edges = [&](int i) {  // edge neighbours not in a run yet
-                int c = 0;
+            // the tile's triangles as sets: their dofs, and their edge neighbours
+            uint64_t dofs[kTileTris], edges[kTileTris] = {};
+            for (int i = 0; i < tc; ++i) {
+                dofs[i] = 0;
+                for (int l = 0; l < 3; ++l) dofs[i] |= 1ull << slot(t0 + i, l);
+            }
+            for (int i = 0; i < tc; ++i)
                 for (int j = 0; j < tc; ++j)
-                    if (j != i && !taken[j] && n_shared(t0 + i, t0 + j) >= 2) ++c;
-                return c;
-            };
+                    if (j != i && __builtin_popcountll(dofs[i] & dofs[j]) >= 2) edges[i] |= 1ull << j;
+            uint64_t taken = 0;
             for (int w0 = 0; w0 < tc; w0 += kRun) {
                 const int n = std::min(kRun, tc - w0), base = t0 + w0;
                 std::vector<int> run;
-                std::vector<char> in_run(kTileMaxDofs, 0);
+                uint64_t in_run = 0, open = 0;
                 while (static_cast<int>(run.size()) < n) {
                     int best = -1, bf = 0, bo = 0;
                     for (int i = 0; i < tc; ++i) {
-                        if (taken[i]) continue;
-                        int fresh = 0;
-                        for (int l = 0; l < 3; ++l) fresh += !in_run[slot(t0 + i, l)];
-                        if (best >= 0 && fresh > bf) continue;
-                        const int oe = open_edges(i);
-                        if (best < 0 || fresh < bf || oe < bo) {
+                        if ((taken >> i) & 1) continue;
+                        const int fresh = __builtin_popcountll(dofs[i] & ~in_run);
+                        const int oe = __builtin_popcountll(edges[i] & ~taken);
+                        if (best < 0 || fresh < bf || (fresh == bf && oe < bo)) {
                             best = i;
                             bf = fresh;
                             bo = oe;
                         }
                     }
-                    taken[best] = 1;
-                    for (int l = 0; l < 3; ++l) in_run[slot(t0 + best, l)] = 1;
-                    run.push_back(t0 + best);
+                    taken |= 1ull << best;
+                    open |= 1ull << best;
+                    in_run |= dofs[best];
+                    run.push_back(best);
                 }
-                std::vector<char> used(static_cast<size_t>(n), 0);
-                auto free_edges = [&](int i) {
-                    int c = 0;
-                    for (int j = 0; j < n; ++j)
-                        if (j != i && !used[j] && n_shared(run[i], run[j]) >= 2) ++c;
-                    return c;
-                };
-                std::vector<int> order;
-                int cur = 0;
-                for (int i = 1; i < n; ++i)
-                    if (free_edges(i) < free_edges(cur)) cur = i;
-                for (int k = 0; k < n; ++k) {
+                std::vector<int> order;  // members of the run
+                int cur = run[0];
+                for (int i : run)
+                    if (__builtin_popcountll(edges[i] & open) < __builtin_popcountll(edges[cur] & open))
+                        cur = i;
+                while (cur >= 0) {
                     order.push_back(cur);
-                    used[cur] = 1;
+                    open &= ~(1ull << cur);
                     int best = -1, bs = -1, bf = 0;
-                    for (int j = 0; j < n; ++j) {
-                        if (used[j]) continue;
-                        const int sh = n_shared(run[cur], run[j]), fe = free_edges(j);
+                    for (int j : run) {
+                        if (!((open >> j) & 1)) continue;
+                        const int sh = __builtin_popcountll(dofs[cur] & dofs[j]);
+                        const int fe = __builtin_popcountll(edges[j] & open);
                         if (sh > bs || (sh == bs && fe < bf)) {
                             best = j;
                             bs = sh;
@@ -626,7 +773,7 @@ std::string build_plan(int nv, int T, int n, int symmetry, const float *vtx, con
                 }
                 int held[3] = {-1, -1, -1};
                 for (int k = 0; k < n; ++k) {
-                    const int p = run[order[k]];
+                    const int p = t0 + order[k];
                     int o[3] = {-1, -1, -1};
                     bool placed[3] = {false, false, false};
                     for (int r = 0; r < 3; ++r)
@@ -727,110 +874,7 @@ std::string build_plan(int nv, int T, int n, int symmetry, const float *vtx, con
             P->tri_i_soa[static_cast<size_t>(j) * T + t] = P->tri_i_aos[static_cast<size_t>(t) * kTriI + j];
     }
 
-    // Singular pair list.
-    std::vector<PairRec> pairs;
-    pairs.reserve(static_cast<size_t>(T) * 16 * M);
-    auto append = [&](int test, int trial, int tm, int sm, Shared s) {
-        int kind;
-        if (s.count == 3) {
-            kind = 1;
-            s.tl1 = 0; s.tl2 = 1; s.sl1 = 0; s.sl2 = 1;
-        } else if (s.count == 2) {
-            kind = 2;
-        } else if (s.count == 1) {
-            kind = 3;
-        } else {
-            return;
-        }
-        pairs.push_back(PairRec{test, trial, tm, sm, kind, s.tl1, s.tl2, s.sl1, s.sl2});
-    };
-    auto shared_by_index = [&](int test, int trial) {
-        Shared s;
-        for (int i = 0; i < 3; ++i)
-            for (int j = 0; j < 3; ++j)
-                if (tri[i * T + test] == tri[j * T + trial]) s.add(i, j);
-        return s;
-    };
-    auto shared_by_key = [&](int test, int trial, int tmi, int smi) {
-        Shared s;
-        const int tm = P->masks[tmi], sm = P->masks[smi];
-        for (int tfl = 0; tfl < 3; ++tfl) {
-            const int tk = key_id(tmi, tri[image_local(tfl, tm) * T + test]);
-            for (int sfl = 0; sfl < 3; ++sfl)
-                if (tk == key_id(smi, tri[image_local(sfl, sm) * T + trial])) s.add(tfl, sfl);
-        }
-        return s;
-    };
-    // Incidence: id -> triangles (CSR), per mask.
-    const int nid = (symmetry == 0) ? nv : static_cast<int>(uniq.size());
-    std::vector<std::vector<int32_t>> start(M), list(M);
-    for (int m = 0; m < (symmetry == 0 ? 1 : M); ++m) {
-        start[m].assign(static_cast<size_t>(nid) + 1, 0);
-        list[m].resize(static_cast<size_t>(T) * 3);
-        auto idof = [&](int t, int l) {
-            const int v = tri[l * T + t];
-            return symmetry == 0 ? v : key_id(m, v);
-        };
-        for (int t = 0; t < T; ++t)
-            for (int l = 0; l < 3; ++l) start[m][idof(t, l) + 1]++;
-        for (int i = 0; i < nid; ++i) start[m][i + 1] += start[m][i];
-        std::vector<int32_t> cur(start[m].begin(), start[m].end() - 1);
-        for (int t = 0; t < T; ++t)
-            for (int l = 0; l < 3; ++l) list[m][cur[idof(t, l)]++] = t;
-    }
-    std::vector<int32_t> stamp(T, 0), cand;
-    int st = 0;
-    for (int trial = 0; trial < T; ++trial) {
-        if (symmetry == 0) {
-            ++st;
-            cand.clear();
-            for (int l = 0; l < 3; ++l) {
-                const int v = tri[l * T + trial];
-                for (int p = start[0][v]; p < start[0][v + 1]; ++p) {
-                    const int test = list[0][p];
-                    if (stamp[test] != st) {
-                        stamp[test] = st;
-                        cand.push_back(test);
-                    }
-                }
-            }
-            for (int test : cand) append(test, trial, 0, 0, shared_by_index(test, trial));
-            continue;
-        }
-        for (int smi = 0; smi < M; ++smi)
-            for (int tmi = 0; tmi < M; ++tmi) {
-                ++st;
-                cand.clear();
-                for (int l = 0; l < 3; ++l) {
-                    const int id = key_id(smi, tri[l * T + trial]);
-                    for (int p = start[tmi][id]; p < start[tmi][id + 1]; ++p) {
-                        const int test = list[tmi][p];
-                        if (stamp[test] != st) {
-                            stamp[test] = st;
-                            cand.push_back(test);
-                        }
-                    }
-                }
-                for (int test : cand) {
-                    const Shared s = (tmi == 0 && smi == 0) ? shared_by_index(test, trial)
-                                                            : shared_by_key(test, trial, tmi, smi);
-                    append(test, trial, P->masks[tmi], P->masks[smi], s);
-                }
-            }
-    }
-    P->kind_count[0] = P->kind_count[1] = P->kind_count[2] = 0;
-    P->image_pairs = 0;
-    std::unordered_set<int64_t> slots;
-    slots.reserve(pairs.size() * 4);
-    for (const PairRec &pr : pairs) {
-        P->kind_count[pr.kind - 1]++;
-        if (pr.tm != 0 || pr.sm != 0) P->image_pairs++;
-        for (int i = 0; i < 3; ++i)
-            for (int j = 0; j < 3; ++j)
-                slots.insert(static_cast<int64_t>(l2g[pr.test * 3 + i]) * n + l2g[pr.trial * 3 + j]);
-    }
-    P->unique_slots = static_cast<int64_t>(slots.size());
-    build_singular_classes(nv, T, vtx, tri, l2g, areas, normals, pairs, P);
+    singular.get();
     P->vtx.assign(vtx, vtx + 3 * (size_t)nv);
     P->tri.assign(tri, tri + 3 * (size_t)T);
     P->normals.assign(normals, normals + 3 * (size_t)T);

@@ -258,3 +258,19 @@ def test_near_quadrature_env_parsing():
     for junk in ("junk", "3", "1:0", "1:-2", "1:inf", "1:nan", "0:1.5", "1:", "1:2:3", " 1"):
         with pytest.raises(RuntimeError, match=NEAR_QUADRATURE_ENV):
             parse({NEAR_QUADRATURE_ENV: junk})
+
+
+@pytest.mark.parametrize("offset", [0, 7, -5])
+def test_open_boundary_edges_are_the_rows_used_once(offset):
+    """Sorted vertex pairs in lexicographic order, whatever the numbering."""
+    from hornlab_metal_bem.mesh import open_boundary_edges
+
+    rng = np.random.default_rng(4)
+    tris = rng.integers(0, 40, (90, 3)) + offset
+    tris = tris[(tris[:, 0] != tris[:, 1]) & (tris[:, 1] != tris[:, 2]) & (tris[:, 0] != tris[:, 2])]
+    edges = np.sort(np.concatenate((tris[:, [0, 1]], tris[:, [1, 2]], tris[:, [2, 0]])), axis=1)
+    rows, counts = np.unique(edges, axis=0, return_counts=True)
+    got = open_boundary_edges(tris)
+    assert got.dtype == np.int32
+    assert np.array_equal(got, rows[counts == 1])
+    assert open_boundary_edges(np.empty((0, 3), np.int32)).shape == (0, 2)
