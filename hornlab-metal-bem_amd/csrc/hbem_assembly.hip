@@ -460,9 +460,9 @@ __device__ __forceinline__ float wave_sum(float x) {
 // One tile pair (pair index tp) at one frequency (b) of the regular
 // assembly: the block body shared by the single-mesh kernel and the
 // multi-mesh launch of a session group.
-template <bool kComplexK, int kM, bool kPrecise>
+template <bool kComplexK, int kM, bool kPrecise, bool kParts>
 __device__ __forceinline__ void regular_tile_pair(
-    const DeviceGeometry &g, int tp, int b, const float *__restrict__ k_real,
+    const DeviceGeometry &g, int tp, int part, int n_parts, int b, const float *__restrict__ k_real,
     const float *__restrict__ k_imag, const float *__restrict__ q, int n_src,
     const float *__restrict__ beta, float *__restrict__ A, int64_t lda, int64_t a_stride,
     float *__restrict__ rhs, int64_t rhs_stride) {
@@ -475,7 +475,12 @@ __device__ __forceinline__ void regular_tile_pair(
     const int s0 = g.tile_start[s_tile], scount = g.tile_count[s_tile], snd = g.tile_ndofs[s_tile];
     const int t0 = g.tile_start[t_tile], tcount = g.tile_count[t_tile];
     const int tnd = g.tile_ndofs[t_tile];
-    const int n_tests = max(0, min(kTestsPerWave, tcount - wave * kTestsPerWave));
+    // this block's share of the wave's run of tests (parts divides 16); without
+    // kParts the whole run, in fewer registers
+    const int parts = kParts ? n_parts : 1;
+    const int run_tests = max(0, min(kTestsPerWave, tcount - wave * kTestsPerWave));
+    const int first = kParts ? part * (kTestsPerWave / parts) : 0;
+    const int n_tests = max(0, min(run_tests - first, kTestsPerWave / parts));
     // the wave's staged values [3][64] and zero slot, then its table
     const int wave_lds = regular_wave_lds(g.run_rows, g.max_tile_dofs);
     v4f *stage = regular_lds + wave * wave_lds;
@@ -551,7 +556,7 @@ __device__ __forceinline__ void regular_tile_pair(
     // access on the per-test path).
     bool tq_lane = false;
     float tbre_lane = 0.0f, tbim_lane = 0.0f;
-    const int rbase = t0 + wave * kTestsPerWave;  // this wave's first test-side record
+    const int rbase = t0 + wave * kTestsPerWave + first;  // the first test-side record
     if (lane < n_tests) {
         const int torig_l = g.tri_t_i[(size_t)(rbase + lane) * kTriI + 19];
         for (int src = 0; src < n_src; ++src) {
@@ -630,7 +635,7 @@ __device__ __forceinline__ void regular_tile_pair(
             for (int c0 = 0; c0 < snd; c0 += 4) {
                 const int c = c0 + (lane >> 4);
                 const int sd = __shfl(col_dof, c);
-                if (r < rows && c < snd) {
+                if (r < rows && c < snd && (!kParts || td >= 0)) {
                     const v4f v = table[r * snd + c];
                     add_to_matrix(td, sd, v[0], v[1]);
                 }
@@ -638,13 +643,15 @@ __device__ __forceinline__ void regular_tile_pair(
         }
         for (int r = 0; r < rows; ++r) {
             const int td = __builtin_amdgcn_readlane(row_dof, r);
+            if (kParts && td < 0) continue;  // a row this share does not use
             if (col_ok) {
                 const v4f v = table[r * snd + lane];
                 add_to_matrix(col_dof, td, v[2], v[3]);
                 table[r * snd + lane] = zero4;
             }
         }
-        if (lane < rows) add_rhs(opaque(rhs_b), row_dof, row_rhs[0], row_rhs[1]);
+        if (lane < rows && (!kParts || row_dof >= 0))
+            add_rhs(opaque(rhs_b), row_dof, row_rhs[0], row_rhs[1]);
         row_rhs[0] = row_rhs[1] = 0.0f;
     };
     int rec = 0;
@@ -792,6 +799,14 @@ __device__ __forceinline__ void regular_tile_pair(
                 flush(r, cur.row[r], cur.dof[r]);
         if (cur.seg > 0) write_table(cur.seg);
     }
+    // a share that ends in an earlier segment than its run: row_map below holds
+    // the last segment's rows
+    if constexpr (kParts) {
+        const int later = first + n_tests + lane;
+        const bool cut = n_tests > 0 && later < run_tests &&
+                         g.tri_t_i[(size_t)(rbase + n_tests + lane) * kTriI + 18] > 0;
+        if (__any(cut)) write_table(g.run_rows);
+    }
     if (col_ok) add_rhs(rhs_b, col_dof, col_rhs[0], col_rhs[1]);
     if (row_dof >= 0) add_rhs(rhs_b, row_dof, row_rhs[0], row_rhs[1]);
     __syncthreads();
@@ -826,13 +841,15 @@ __device__ __forceinline__ void regular_tile_pair(
     }
 }
 
-template <bool kComplexK, int kM, bool kPrecise>
+template <bool kComplexK, int kM, bool kPrecise, bool kParts>
 __global__ __launch_bounds__(256, 2) void k_assemble_regular(
-    DeviceGeometry g, const float *__restrict__ k_real, const float *__restrict__ k_imag,
-    const float *__restrict__ q, int n_src, const float *__restrict__ beta,
-    float *__restrict__ A, int64_t lda, int64_t a_stride, float *__restrict__ rhs,
-    int64_t rhs_stride) {
-    regular_tile_pair<kComplexK, kM, kPrecise>(g, blockIdx.x, blockIdx.y, k_real, k_imag, q, n_src,
+    DeviceGeometry g, int parts, const float *__restrict__ k_real,
+    const float *__restrict__ k_imag, const float *__restrict__ q, int n_src,
+    const float *__restrict__ beta, float *__restrict__ A, int64_t lda, int64_t a_stride,
+    float *__restrict__ rhs, int64_t rhs_stride) {
+    regular_tile_pair<kComplexK, kM, kPrecise, kParts>(
+        g, kParts ? blockIdx.x / parts : blockIdx.x, kParts ? blockIdx.x % parts : 0, parts,
+        blockIdx.y, k_real, k_imag, q, n_src,
                                                beta, A, lda, a_stride, rhs, rhs_stride);
 }
 
@@ -856,7 +873,7 @@ __global__ __launch_bounds__(256, 2) void k_assemble_regular_multi(
     const AssemblyJob &jb = jobs[j];
     const int local = blockIdx.x - jb.block_begin_reg;
     const int ntp = jb.g.n_tile_pairs;
-    regular_tile_pair<kComplexK, kM, false>(jb.g, local % ntp, local / ntp, jb.k_real, jb.k_imag,
+    regular_tile_pair<kComplexK, kM, false, false>(jb.g, local % ntp, 0, 1, local / ntp, jb.k_real, jb.k_imag,
                                             jb.q, jb.n_src, jb.beta, jb.A, jb.lda, jb.a_stride,
                                             jb.rhs, jb.rhs_stride);
 }
@@ -1542,17 +1559,29 @@ void launch_assemble_regular(const DeviceGeometry &g, int n_batch, const float *
                              float *A, int64_t lda, int64_t a_stride, float *rhs,
                              int64_t rhs_stride, hipStream_t stream, bool precise) {
     if (g.n_tile_pairs == 0 || n_batch <= 0) return;
-    dim3 grid(g.n_tile_pairs, n_batch);
+    // Two blocks fit a CU.  A launch of a few rounds loses most of its last one,
+    // and one of less than a round leaves CUs idle: its blocks are cut in two or
+    // four (each then writes its rows to A on its own): 528 blocks (1078 dofs, one
+    // frequency) 0.505 ms whole, 0.422 in four.  The FP64-geometry variant runs
+    // whole (registers).
+    const int64_t blocks = (int64_t)g.n_tile_pairs * n_batch;
+    const int parts = precise || blocks >= 2048 ? 1 : (blocks >= 1024 ? 2 : 4);
+    dim3 grid(g.n_tile_pairs * parts, n_batch);
     const size_t shm = 64 * (size_t)regular_wave_lds(g.run_rows, g.max_tile_dofs);
     auto go = [&](auto complex_k, auto masks) {
         constexpr bool kC = decltype(complex_k)::value;
         constexpr int kM = decltype(masks)::value;
         if (precise)
-            hipLaunchKernelGGL((k_assemble_regular<kC, kM, true>), grid, dim3(256), shm, stream, g,
-                               k_real, k_imag, q, n_src, beta, A, lda, a_stride, rhs, rhs_stride);
+            hipLaunchKernelGGL((k_assemble_regular<kC, kM, true, false>), grid, dim3(256), shm, stream, g,
+                               parts, k_real, k_imag, q, n_src, beta, A, lda, a_stride, rhs,
+                               rhs_stride);
+        else if (parts > 1)
+            hipLaunchKernelGGL((k_assemble_regular<kC, kM, false, true>), grid, dim3(256), shm,
+                               stream, g, parts, k_real, k_imag, q, n_src, beta, A, lda, a_stride,
+                               rhs, rhs_stride);
         else
-            hipLaunchKernelGGL((k_assemble_regular<kC, kM, false>), grid, dim3(256), shm, stream,
-                               g, k_real, k_imag, q, n_src, beta, A, lda, a_stride, rhs,
+            hipLaunchKernelGGL((k_assemble_regular<kC, kM, false, false>), grid, dim3(256), shm, stream,
+                               g, parts, k_real, k_imag, q, n_src, beta, A, lda, a_stride, rhs,
                                rhs_stride);
     };
     auto by_masks = [&](auto complex_k) {

@@ -113,6 +113,23 @@ def test_split_and_whole_singular_rules_agree(require_gpu):
             assert rel_l2(one[0].pressure, whole[i].pressure) < 2e-5
 
 
+@pytest.mark.parametrize("n_freq", [200, 400])
+def test_whole_halved_and_quartered_runs_agree(require_gpu, n_freq):
+    """Six tile pairs per frequency: one frequency cuts the blocks in four, 200
+    in two, 400 not at all, with tables that overflow in each."""
+    b = _soup(37)
+    f = np.geomspace(300.0, 1500.0, n_freq)
+    k = (2 * np.pi * f / 343.0).astype(np.float32)
+    q = np.ones((n_freq, b.n_triangles), np.complex64)
+    obs = np.array([[0.0], [0.0], [2.0]], np.float32)
+    with _session(b) as s:
+        batch = s.assemble_solve_evaluate_standard_neumann_batch(f, k, q, obs)
+        for i in (0, n_freq // 2, n_freq - 1):
+            one = s.assemble_solve_evaluate_standard_neumann_batch(f[i:i + 1], k[i:i + 1], q[i:i + 1], obs)
+            # FP32 rounding times cond (separate triangles: below 100)
+            assert rel_l2(batch[i].pressure, one[0].pressure) < 2e-5
+
+
 @pytest.mark.parametrize("plane", [None, "yz+xz"])
 @pytest.mark.parametrize("n_obs", [1, 63, 64, 65, 257])
 def test_field_points_near_and_far(require_gpu, plane, n_obs):
