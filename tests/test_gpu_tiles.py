@@ -130,6 +130,16 @@ def test_whole_halved_and_quartered_runs_agree(require_gpu, n_freq):
             assert rel_l2(batch[i].pressure, one[0].pressure) < 2e-5
 
 
+def _field_terms(b, p, q, obs):
+    """Sum of the magnitudes of the identity image's field terms per point."""
+    X, Y, W = O.rule6()
+    v = b.vertices_3xn_f32[:, b.triangles_3xm_i32].astype(float)  # (3, 3, T)
+    y = np.einsum("bl,clt->cbt", np.stack([1 - X - Y, X, Y], 1), v)
+    r = np.linalg.norm(y[:, :, :, None] - obs[:, None, None, :], axis=0)
+    w = W[:, None, None] * (2 * b.triangle_areas_f32)[None, :, None] / (4 * np.pi)
+    return (w * (np.abs(p).max() / r ** 2 + np.abs(q)[None, :, None] / r)).sum((0, 1))
+
+
 @pytest.mark.parametrize("plane", [None, "yz+xz"])
 @pytest.mark.parametrize("n_obs", [1, 63, 64, 65, 257])
 def test_field_points_near_and_far(require_gpu, plane, n_obs):
@@ -148,18 +158,37 @@ def test_field_points_near_and_far(require_gpu, plane, n_obs):
         got = s.evaluate_standard_exterior_batch(np.array([1000.0]), k, p[None], q[None], obs)[0]
     want = O.field(O.Geometry.from_buffers(b, plane), 20.0, p, q, obs)
     # near points: each term |p| jac w / (4 pi r^2) + |q| jac w / (4 pi r) of
-    # the sum carries about ten roundings of 6e-8 (its distance, formed from a
-    # vertex and an offset up to 30 times as long, more than its product), so
-    # 4e-6 of the terms' sum bounds the error (the identity image's terms; the
-    # others are farther)
-    X, Y, W = O.rule6()
-    v = b.vertices_3xn_f32[:, b.triangles_3xm_i32].astype(float)  # (3, 3, T)
-    y = np.einsum("bl,clt->cbt", np.stack([1 - X - Y, X, Y], 1), v)
-    r = np.linalg.norm(y[:, :, :, None] - obs[:, None, None, ::4], axis=0)
-    w = W[:, None, None] * (2 * b.triangle_areas_f32)[None, :, None] / (4 * np.pi)
-    terms = (w * (np.abs(p).max() / r ** 2 + np.abs(q)[None, :, None] / r)).sum((0, 1))
+    # the sum carries about ten roundings of 6e-8, and a few dozen the partial
+    # sums, so 4e-6 of the terms' sum bounds the error (the identity image's
+    # terms; the others are farther)
+    terms = _field_terms(b, p, q, obs[:, ::4])
     assert np.all(np.abs(got - want)[::4] < 4e-6 * terms)
     far = np.ones(n_obs, bool)
     far[::4] = False
     if far.any():
         assert rel_l2(got[far], want[far]) < 5e-6
+
+
+@pytest.mark.parametrize("plane", [None, "yz+xz"])
+def test_field_points_close_to_the_surface(require_gpu, plane):
+    """Points 0.05 to 20 mm off 30 mm triangles, over any of their points: the
+    nearest quadrature point is up to hundreds of times closer than the
+    triangle is wide, and its distance still has to be good to FP32."""
+    b = horn_buffers(edge_length=0.03, quarter=plane is not None)
+    rng = np.random.default_rng(5)
+    n_obs, X, Y = 400, *O.rule6()[:2]
+    tri = rng.integers(0, b.n_triangles, n_obs)
+    at = rng.dirichlet([1, 1, 1], n_obs)
+    a = rng.integers(0, 6, n_obs // 2)
+    at[::2] = np.stack([1 - X - Y, X, Y], 1)[a]  # straight above a quadrature point
+    v = b.vertices_3xn_f32[:, b.triangles_3xm_i32[:, tri]].astype(float)
+    off = np.geomspace(5e-5, 2e-2, n_obs) * b.triangle_normals_3xm_f32[:, tri]
+    obs = (np.einsum("ol,clo->co", at, v) - off).astype(np.float32)
+    p = (rng.standard_normal(b.p1_dof_count) + 1j * rng.standard_normal(b.p1_dof_count)).astype(np.complex64)
+    q = (20 * rng.standard_normal(b.n_triangles)).astype(np.complex64)
+    with _session(b, plane) as s:
+        got = s.evaluate_standard_exterior_batch(
+            np.array([1000.0]), np.array([20.0], np.float32), p[None], q[None], obs)[0]
+    want = O.field(O.Geometry.from_buffers(b, plane), 20.0, p, q, obs)
+    # about ten roundings of 6e-8 per term
+    assert np.all(np.abs(got - want) < 6e-7 * _field_terms(b, p, q, obs))
