@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from hornlab_metal_bem.procedural import HornSpec
 from meshes import buffers_from_arrays, horn_buffers, mesh_buffers, rel_l2, sphere_buffers
 
 pytestmark = pytest.mark.gpu
@@ -79,6 +80,26 @@ def test_long_column_lists(require_gpu, valence):
 def test_quarter_horn_all_sources_and_walls(require_gpu, edge, plane):
     _check_assembly(horn_buffers(edge_length=edge), plane, 60.0)
     _check_assembly(horn_buffers(edge_length=edge), plane, 60.0, 0.5, 0.3 - 0.2j)
+
+
+def test_entries_of_distant_pairs_at_a_high_wavenumber(require_gpu):
+    """k = 300 1/m on a mesh of 8.9 mm edges: an entry is a sum of over a
+    thousand evaluations whose own roundings (phase errors of 4e-6, r times
+    roundings of 6e-8 times k) average out, so what it keeps is what they
+    share.  8.5e-7 admits the point offset of a test triangle rounded with its
+    vertex difference (7.5e-7), not the vertex difference rounded by itself
+    as well (9.4e-7)."""
+    b = horn_buffers(edge_length=0.0089, seed=2, spec=HornSpec(0.0127, 0.150, 0.150, 0.020, "exponential"))
+    q = np.ones(b.n_triangles, np.complex64)
+    with _session(b, "yz+xz") as s:
+        A, _ = s.assemble_standard_neumann(0.0, 300.0, q)
+    Ao, _, _ = O.assemble(O.Geometry.from_buffers(b, "yz+xz"), 300.0, q)
+    far = np.ones(A.shape, bool)  # entries whose dofs share no triangle
+    dofs = b.p1_local2global_i32.reshape(-1, 3)
+    for i in range(3):
+        for j in range(3):
+            far[dofs[:, i], dofs[:, j]] = False
+    assert rel_l2(A[far], Ao[far]) < 8.5e-7
 
 
 @pytest.mark.parametrize("n_sources", [1, 2, 3])
