@@ -262,6 +262,10 @@ __device__ __forceinline__ void unpack_test(int w, TestRec &r) {
     r.dev = i(23);
 }
 
+// Beyond any mesh, and near enough for a finite r^2 and a phase within the
+// range of the hardware sine.
+constexpr float kSkippedAt = 1.0e6f;
+
 // One (t, s) over all images and both directions: tr is t's record (uniform),
 // yo / v0s / ns the lane's trial points (offsets from vertex 0), vertex 0 and
 // normal.  Adds jac_t times the block sums over the 6 x 6 rule to
@@ -281,7 +285,8 @@ __device__ __forceinline__ void unpack_test(int w, TestRec &r) {
 //   d . n_s       = (v0_s - S_m x_a) . n_s    = hF[a]
 //   d . (S_m n_t) = (y_b - S_m v0_t) . (S_m n_t) = hR[b]
 // Only non-touching combinations count, so r > 0; a skipped lane's triangle is
-// moved 1000 m away, which keeps it finite, and its factors are zero.
+// moved far away and loses its damping (which grows with the distance where
+// k_imag < 0), so its terms stay finite, and its factors are zero.
 //
 // Loop order: test points outer, images inner, trial points innermost, so the
 // sums over t's basis weights are formed once per test point for all images,
@@ -311,7 +316,7 @@ __device__ __forceinline__ void regular_pair(const TestRec &tr, int packed_masks
                 const float lost = v0s[c] - (dv[m][c] + (v0s[c] - dv[m][c]));
                 dl[m][c] = lost + ((v0s[c] - dv[m][c]) - v0t);
             }
-            if (c == 0 && on[m] == 0.0f) dv[m][c] = (DT)1.0e3f;
+            if (c == 0 && on[m] == 0.0f) dv[m][c] = (DT)kSkippedAt;
             dvf[c] = (float)dv[m][c];
         }
         const float cR = -on[m] * rf * tr.jac;
@@ -351,7 +356,8 @@ __device__ __forceinline__ void regular_pair(const TestRec &tr, int packed_masks
                 (on[m] * tr.jac);
             BasisSum<!kPrecise> em;  // this image's sums before hF
             em.clear();
-// distances of the six points, then their transcendentals as one
+            const float damping = kComplexK ? -kim * on[m] : 0.0f;
+            // distances of the six points, then their transcendentals as one
             // run at raised wave priority (below), then the sums
             DT r2d[6];
             float rinv[6], rr[6], sn[6], cs[6];
@@ -388,7 +394,7 @@ __device__ __forceinline__ void regular_pair(const TestRec &tr, int packed_masks
             for (int bq = 0; bq < 6; ++bq) {
                 cs[bq] = __builtin_amdgcn_cosf(sn[bq]);
                 sn[bq] = __builtin_amdgcn_sinf(sn[bq]);
-                if (kComplexK) rr[bq] = __expf(-kim * rr[bq]);  // damping
+                if (kComplexK) rr[bq] = __expf(damping * rr[bq]);
             }
             trans_end();
 #pragma unroll

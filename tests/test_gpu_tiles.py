@@ -213,3 +213,29 @@ def test_field_points_close_to_the_surface(require_gpu, plane):
     want = O.field(O.Geometry.from_buffers(b, plane), 20.0, p, q, obs)
     # about ten roundings of 6e-8 per term
     assert np.all(np.abs(got - want) < 6e-7 * _field_terms(b, p, q, obs))
+
+
+@pytest.mark.parametrize("precise", [False, True])
+@pytest.mark.parametrize("plane", [None, "yz+xz"])
+def test_growing_waves_stay_finite(require_gpu, plane, precise):
+    """Device arrays may hold k_imag < 0 (the host entry points refuse it):
+    e^{-k_imag r} then grows with the distance, which must not reach the lanes
+    whose pair is left out."""
+    import torch
+
+    b = horn_buffers(edge_length=0.03, quarter=plane is not None)
+    k, kim = 20.0, -0.25
+    q = (b.physical_tags_i32 == 2).astype(np.complex64)
+    dev = {n: torch.as_tensor(a, device="cuda:0") for n, a in dict(
+        k=np.array([k], np.float32), kim=np.array([kim], np.float32), q=q[None],
+        obs=np.array([[0.1], [0.2], [2.0]], np.float32)).items()}
+    field = torch.zeros(1, dtype=torch.complex64, device="cuda:0")
+    p = torch.zeros(b.p1_dof_count, dtype=torch.complex64, device="cuda:0")
+    tag = torch.zeros(2, dtype=torch.complex128, device="cuda:0")
+    with _session(b, plane) as s:
+        s.solve_batch_device(1, dev["k"].data_ptr(), dev["k"].data_ptr(), dev["q"].data_ptr(), 1,
+                             dev["obs"].data_ptr(), field.data_ptr(), tag.data_ptr(),
+                             k_imag_ptr=dev["kim"].data_ptr(), p_ptr=p.data_ptr(), source_tags=[2],
+                             precise_geometry=precise)
+    A, rhs, _ = O.assemble(O.Geometry.from_buffers(b, plane), k, q, kim=kim)
+    assert rel_l2(p.cpu().numpy(), O.solve(A, rhs)) < 2e-5  # cond(A) ~ 30
