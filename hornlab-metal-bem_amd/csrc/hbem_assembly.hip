@@ -284,7 +284,8 @@ constexpr float kSkippedAt = 1.0e6f;
 // are flat, so the normal projections of d depend on one point only:
 //   d . n_s       = (v0_s - S_m x_a) . n_s    = hF[a]
 //   d . (S_m n_t) = (y_b - S_m v0_t) . (S_m n_t) = hR[b]
-// Only non-touching combinations count, so r > 0; a skipped lane's triangle is
+// Only non-touching combinations count, so r > 0 unless points of triangles
+// without a common vertex coincide; a skipped lane's triangle is
 // moved far away and loses its damping (which grows with the distance where
 // k_imag < 0), so its terms stay finite, and its factors are zero.
 //
@@ -371,10 +372,15 @@ __device__ __forceinline__ void regular_pair(const TestRec &tr, int packed_masks
             trans_begin();
 #pragma unroll
             for (int bq = 0; bq < 6; ++bq) rinv[bq] = __builtin_amdgcn_rsqf((float)r2d[bq]);
+            if constexpr (kPrecise) {
+                // points of triangles that share no vertex may coincide: no
+                // term, as in the gradient's kernels
+#pragma unroll
+                for (int bq = 0; bq < 6; ++bq) rinv[bq] = r2d[bq] > 1.0e-14 ? rinv[bq] : 0.0f;
+            }
 #pragma unroll
             for (int bq = 0; bq < 6; ++bq) {
-                const float r2 = (float)r2d[bq];
-                const float r = r2 * rinv[bq];
+                const float r = (float)r2d[bq] * rinv[bq];
                 if (kComplexK) rr[bq] = r;
                 float t;  // revolutions
                 if constexpr (kPrecise) {

@@ -239,3 +239,20 @@ def test_growing_waves_stay_finite(require_gpu, plane, precise):
                              precise_geometry=precise)
     A, rhs, _ = O.assemble(O.Geometry.from_buffers(b, plane), k, q, kim=kim)
     assert rel_l2(p.cpu().numpy(), O.solve(A, rhs)) < 2e-5  # cond(A) ~ 30
+
+
+def test_coincident_points_with_fp64_geometry(require_gpu):
+    """A triangle given twice, with vertices and dofs of its own each time:
+    no common index, so the pair is regular and six distances are zero, which
+    add nothing (as in the oracle)."""
+    one = _soup(12)
+    V = np.concatenate([one.vertices_3xn_f32, one.vertices_3xn_f32[:, :3]], axis=1)
+    E = np.arange(39).reshape(13, 3)
+    b = buffers_from_arrays(V, E.T, E, 39, np.full(13, 2))
+    q = np.ones((1, 13), np.complex64)
+    with _session(b) as s:
+        r = s.assemble_solve_evaluate_standard_neumann_batch(
+            np.array([1000.0]), np.array([20.0], np.float32), q, np.array([[0.0], [0.0], [2.0]], np.float32),
+            precise_geometry=True)[0]
+    A, rhs, _ = O.assemble(O.Geometry.from_buffers(b), 20.0, q[0])
+    assert rel_l2(r.pressure, O.solve(A, rhs)) < 2e-5  # cond(A) below 100
