@@ -176,6 +176,8 @@ struct hbem_session {
     DevBuf lu_perm, lu_pi, lu_lf, lu_dinv, ts_ctx[2], ts_y[2], ts_z[2];
     hbem::TrsvSync trsv[2] = {};
     bool trsv_on = false;
+    uint32_t *trsv_expired = nullptr;  // [2], pinned
+    uint32_t trsv_polls = hbem::kTrsvPolls;
     double setup_seconds = 0.0;
     int64_t near_pairs = 0;
     int assembly_mode = HBEM_ASSEMBLY_CORRECTED;
@@ -191,6 +193,7 @@ struct hbem_session {
                           &ts_ctx[1], &ts_y[0], &ts_y[1], &ts_z[0], &ts_z[1]})
             b->release();
         if (lu_graph) (void)hipGraphExecDestroy(lu_graph);
+        if (trsv_expired) (void)hipHostFree(trsv_expired);
         if (aux_stream) (void)hipStreamDestroy(aux_stream);
         if (ev_lu) (void)hipEventDestroy(ev_lu);
         if (stream) (void)hipStreamDestroy(stream);
@@ -299,10 +302,27 @@ hbem::TrsvSync trsv_sync(hbem_session *s, int which, int V, int N, hipStream_t s
     c.reserve(sizeof(uint32_t) * 4);
     y.reserve(sizeof(uint64_t) * words);
     z.reserve(sizeof(uint64_t) * words);
-    const hbem::TrsvSync sync{c.as<uint32_t>(), y.as<uint64_t>(), z.as<uint64_t>()};
+    if (!s->trsv_expired) {
+        void *host = nullptr;
+        hip_check(hipHostMalloc(&host, 2 * sizeof(uint32_t), hipHostMallocDefault), "hipHostMalloc");
+        s->trsv_expired = static_cast<uint32_t *>(host);
+    }
+    s->trsv_expired[which] = 0;
+    const hbem::TrsvSync sync{c.as<uint32_t>(), y.as<uint64_t>(), z.as<uint64_t>(),
+                              s->trsv_expired + which, s->trsv_polls};
     if (c.ptr != c0 || y.ptr != y0 || z.ptr != z0)
         hbem::launch_trsv_init(sync, std::min(y.bytes, z.bytes) / sizeof(uint64_t), st);
     return sync;
+}
+
+// After the stream of solve context `which` has been waited for: fails if a
+// wait between the workgroups of one of its solves ran out (the values are NaN).
+void check_trsv(hbem_session *s, int which) {
+    if (!s->trsv_on) return;
+    volatile uint32_t *expired = s->trsv_expired + which;
+    if (*expired == 0) return;
+    *expired = 0;
+    fail(HBEM_EHIP, "a wait between the workgroups of a triangular solve ran out");
 }
 
 // Runs on `st`; its buffers come from reserve_rcond (no allocation here, so
@@ -342,6 +362,7 @@ void estimate_rcond(hbem_session *s, const hbem::LuWorkspace &w, std::vector<dou
                              st),
               "rcond D2H");
     hip_check(hipStreamSynchronize(st), "rcond sync");
+    check_trsv(s, 1);
 }
 
 }  // namespace
@@ -557,6 +578,15 @@ int32_t hbem_session_set_assembly_mode(hbem_session *s, int32_t mode) {
         }
         s->assembly_mode = mode;
         s->adj_valid = false;
+    });
+}
+
+int32_t hbem_session_set_wait_limit(hbem_session *s, uint32_t polls) {
+    return guarded([&] {
+        if (!s) fail(HBEM_EINVAL, "hbem_session_set_wait_limit: null session");
+        std::lock_guard<std::mutex> lock(s->mu);
+        s->trsv_polls = polls ? polls : hbem::kTrsvPolls;
+        for (hbem::TrsvSync &t : s->trsv) t.polls = s->trsv_polls;
     });
 }
 
@@ -1119,7 +1149,8 @@ void solve_resident(hbem_session *s, int B, int S, int n, int N, const hbem_solv
             (uintptr_t)s->info.ptr, (uintptr_t)s->gl.ptr, (uintptr_t)s->lu_scr_i.ptr,
             (uintptr_t)s->lu_scr_f.ptr, (uintptr_t)s->anorm.ptr, (uintptr_t)s->amax.ptr,
             (uintptr_t)s->lu_scale.ptr, (uintptr_t)w.pack, (uintptr_t)w.perm, (uintptr_t)w.pi, (uintptr_t)w.dinv, (uintptr_t)w.lf,
-            (uintptr_t)s->ts_ctx[0].ptr, (uintptr_t)s->ts_y[0].ptr, (uintptr_t)s->ts_z[0].ptr};
+            (uintptr_t)s->ts_ctx[0].ptr, (uintptr_t)s->ts_y[0].ptr, (uintptr_t)s->ts_z[0].ptr,
+            (uintptr_t)s->trsv_polls};
         if (!s->lu_graph || s->lu_graph_key != key) {
             if (s->lu_graph) {
                 (void)hipGraphExecDestroy(s->lu_graph);
@@ -1279,6 +1310,7 @@ void solve_resident(hbem_session *s, int B, int S, int n, int N, const hbem_solv
     }
     t.stop(st);
     *solve_seconds = t.seconds();
+    check_trsv(s, 0);
     if (after_solve) after_solve();
     if (rc_thread.joinable()) rc_thread.join();
     if (rc_error) std::rethrow_exception(rc_error);
@@ -1717,6 +1749,7 @@ int32_t hbem_adjoint_backward(hbem_session *s, const float *grad_field, double *
                                     s->adj_sig.as<double>(), grad_q, st);
         hip_check(hipGetLastError(), "adjoint launch");
         hip_check(hipStreamSynchronize(st), "adjoint sync");
+        check_trsv(s, 0);
     });
 }
 

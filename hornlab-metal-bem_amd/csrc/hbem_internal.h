@@ -438,16 +438,21 @@ inline int lu_solve_blocks(int N) { return (N + kLuOuter - 1) / kLuOuter; }
 inline size_t lu_dinv_floats(int N) { return (size_t)N * 64 * 2 * 2; }
 
 // Synchronisation state of the multi-workgroup triangular solves of one
-// stream (orders <= kTrsvMaxOrder): ctx[4] = {ticket, finished blocks,
-// epoch, error}; y and z [V][N][2] epoch-tagged words of the forward and
+// stream (orders <= kTrsvMaxOrder): ctx[3] = {ticket, finished blocks,
+// epoch}; y and z [V][N][2] epoch-tagged words of the forward and
 // backward values.  Set up once by launch_trsv_init (y and z cleared over
 // n_words words each); a context serves one stream at a time (launches on it
-// are ordered).
+// are ordered).  A wait takes at most `polls` polls; past that the values are
+// NaN and *expired, in host memory the device can write, is set: the host
+// reads it once the stream has been waited for.
 struct TrsvSync {
     uint32_t *ctx;
     uint64_t *y;
     uint64_t *z;
+    uint32_t *expired;
+    uint32_t polls;
 };
+constexpr uint32_t kTrsvPolls = 1u << 20;
 inline size_t trsv_words(int V, int N) { return (size_t)V * N * 2; }
 void launch_trsv_init(const TrsvSync &sync, size_t n_words, hipStream_t stream);
 

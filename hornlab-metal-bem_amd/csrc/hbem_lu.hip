@@ -1591,9 +1591,8 @@ __global__ __launch_bounds__(1024) void k_lu_solve(const float *A, int64_t lda, 
 // wait sits between producer and consumer.  A workgroup takes its panel from
 // a ticket counter in arrival order and waits only on panels with smaller
 // tickets, which belong to workgroups already running, so every wait ends
-// without co-residency of the grid; each wait is also bounded (kTrsvSpin
-// polls): past it the panel goes on with NaN values and sets the context's
-// error word.
+// without co-residency of the grid; each wait is also bounded (sync.polls):
+// past it the panel goes on with NaN values and sets *sync.expired.
 // Rows are in the final order of the factorization (all exchanges applied).
 // The L columns of outer block s are stored in the row order at the end of
 // block s; k_lu_final_l copies L once per factorization into final row order
@@ -1606,12 +1605,11 @@ __global__ __launch_bounds__(1024) void k_lu_solve(const float *A, int64_t lda, 
 // tagged words).
 // ---------------------------------------------------------------------------
 constexpr int kTrsvRows = 64;
-constexpr uint32_t kTrsvSpin = 1u << 20;
 static_assert(kLuOuter % kTrsvRows == 0 && kLuPad % kTrsvRows == 0, "panels inside outer blocks");
 
 __global__ void k_trsv_init(uint32_t *ctx, uint64_t *y, uint64_t *z, size_t n_words) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < 4) ctx[i] = i == 2 ? 1u : 0u;  // ticket, finished, epoch 1, error
+    if (i < 3) ctx[i] = i == 2 ? 1u : 0u;  // ticket, finished, epoch 1
     if (i < n_words) {
         y[i] = 0ull;  // epoch 0: never current
         z[i] = 0ull;
@@ -1841,7 +1839,7 @@ __global__ __launch_bounds__(256) void k_trsv(const float *A, const float *lf, i
                 re = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 im = __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if (__all(word_epoch(re) == ep && word_epoch(im) == ep)) break;
-                if (!ok || i + 1 >= kTrsvSpin) {
+                if (!ok || i + 1 >= sync.polls) {
                     ok = false;
                     break;
                 }
@@ -1940,7 +1938,8 @@ __global__ __launch_bounds__(256) void k_trsv(const float *A, const float *lf, i
     }
     __syncthreads();
     if (tid == 0) {
-        if (!ok) atomicOr(&sync.ctx[3], 1u);
+        if (!ok)
+            __hip_atomic_store(sync.expired, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         // the last workgroup resets the ticket counter and opens the next epoch
         if (atomicAdd(&sync.ctx[1], 1u) == gridDim.x - 1) {
             __hip_atomic_store(&sync.ctx[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

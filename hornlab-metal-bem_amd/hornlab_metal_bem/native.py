@@ -150,6 +150,7 @@ EXPORTED_SYMBOLS = (
     "hbem_session_get_info",
     "hbem_session_set_near_field",
     "hbem_session_set_assembly_mode",
+    "hbem_session_set_wait_limit",
     "hbem_assemble",
     "hbem_solve_batch",
     "hbem_solve_batch_device",
@@ -251,6 +252,8 @@ def load_library() -> C.CDLL:
         lib.hbem_session_set_near_field.restype = C.c_int32
         lib.hbem_session_set_assembly_mode.argtypes = [C.c_void_p, C.c_int32]
         lib.hbem_session_set_assembly_mode.restype = C.c_int32
+        lib.hbem_session_set_wait_limit.argtypes = [C.c_void_p, C.c_uint32]
+        lib.hbem_session_set_wait_limit.restype = C.c_int32
         fp = C.POINTER(C.c_float)
         lib.hbem_assemble.argtypes = [C.c_void_p, C.c_float, C.c_float, fp, fp, fp, fp, fp, fp, fp, fp]
         lib.hbem_assemble.restype = C.c_int32

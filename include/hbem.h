@@ -211,6 +211,11 @@ int32_t hbem_session_set_near_field(hbem_session *session, int32_t level, double
 #define HBEM_ASSEMBLY_REGULAR 1
 int32_t hbem_session_set_assembly_mode(hbem_session *session, int32_t mode);
 
+/* Polls after which a workgroup of a triangular solve stops waiting for
+ * another one (0: the default, about a second).  A solve in which that
+ * happens fails with HBEM_EHIP. */
+int32_t hbem_session_set_wait_limit(hbem_session *session, uint32_t polls);
+
 int32_t hbem_session_get_info(hbem_session *session, hbem_session_info *info);
 
 /* Assemble the corrected standard-Neumann system at one wavenumber:

@@ -188,3 +188,46 @@ def test_optimized_mode_in_batch_diagnostics(require_gpu):
     p_ref = O.solve(A_ref, rhs_ref)
     assert rel_l2(res[0].pressure, p_ref) < 1e-4, rel_l2(res[0].pressure, p_ref)
     assert T == q.shape[1]
+
+
+def test_solves_whose_waits_run_out_are_errors(require_gpu):
+    """With one poll per wait the eleven panels of a 642-dof solve cannot hand
+    their values on: the forward, CHIEF and gradient solves say so instead of
+    returning the NaN, and the session works again with the default limit."""
+    import torch
+    from meshes import sphere_buffers
+
+    from hornlab_metal_bem.native import HipBemSession, load_library
+
+    b = sphere_buffers(subdivisions=3)
+    k = np.array([10.0], np.float32)
+    q = np.ones((1, b.n_triangles), np.complex64)
+    obs = np.array([[0.0], [0.0], [2.0]], np.float32)
+    limit = load_library().hbem_session_set_wait_limit
+    expired = pytest.raises(RuntimeError, match="wait between the workgroups")
+    with HipBemSession.create_session(b) as s:
+        def solve(**kw):
+            return s.assemble_solve_evaluate_standard_neumann_batch(np.array([546.0]), k, q, obs, **kw)[0]
+
+        chief = dict(chief_points=np.array([[0.01], [0.02], [0.0]], np.float32))
+        want = solve(estimate_rcond=False).pressure
+        for kw in (dict(estimate_rcond=False), dict(estimate_rcond=True), dict(solve_mode="mixed_fp16"), chief):
+            assert limit(s._handle, 1) == 0
+            with expired:
+                solve(**kw)
+            assert limit(s._handle, 0) == 0
+            assert rel_l2(solve(**kw).pressure, want) < 1e-4
+        dk, dq = torch.as_tensor(k, device="cuda:0"), torch.as_tensor(q, device="cuda:0")
+        do = torch.as_tensor(obs, device="cuda:0")
+        field = torch.zeros((1, 1), dtype=torch.complex64, device="cuda:0")
+        tag = torch.zeros((1, 1), dtype=torch.complex128, device="cuda:0")
+        grad = torch.zeros((3, b.n_vertices), dtype=torch.float64, device="cuda:0")
+        one = torch.ones((1, 1), dtype=torch.complex64, device="cuda:0")
+        s.adjoint_forward_device(1, dk.data_ptr(), dk.data_ptr(), dq.data_ptr(), 1, do.data_ptr(),
+                                 field.data_ptr(), tag.data_ptr(), source_tags=[2])
+        limit(s._handle, 1)
+        with expired:
+            s.adjoint_backward_device(one.data_ptr(), grad.data_ptr())
+        limit(s._handle, 0)
+        s.adjoint_backward_device(one.data_ptr(), grad.data_ptr())
+        assert bool(torch.isfinite(grad).all()) and float(grad.abs().max()) > 0.0
