@@ -1344,11 +1344,17 @@ int batch_size_for(const hbem_session *s, int F, int N, const hbem_solve_options
     if (opt.batch_frequencies > 0) return std::min(F, opt.batch_frequencies);
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = (size_t)16 << 30;
-    const bool refine = opt.solve_mode != HBEM_SOLVE_F32;
+    const bool refine = opt.solve_mode != HBEM_SOLVE_F32 || opt.n_chief > 0;
+    const bool trsv = N <= hbem::kTrsvMaxOrder;
+    const double S = std::max(1, (int)opt.n_sources), m = std::max(0, (int)opt.n_chief);
     // A, the refinement's copy of A, L in final row order for the
-    // multi-workgroup solves, the 16-bit LU operands
-    const double mats = 1.0 + (refine ? 1.0 : 0.0) + (N <= hbem::kTrsvMaxOrder ? 1.0 : 0.0);
-    const double per = (double)N * N * 8.0 * mats + (double)N * 64.0 +
+    // multi-workgroup solves, the 16-bit LU operands; per vector the
+    // right-hand side, the solution and three FP64 vectors; per CHIEF row the
+    // row, its solve and three FP64 vectors; the solve context's words of
+    // either
+    const double mats = 1.0 + (refine ? 1.0 : 0.0) + (trsv ? 1.0 : 0.0);
+    const double per = (double)N * N * 8.0 * mats + (double)N * 64.0 * (S + m) +
+                       (trsv ? (double)N * 32.0 * std::max(S, m) : 0.0) +
                        (refine ? 2.0 * (double)hbem::lu_pack_u16(N) : 0.0);
     const double budget = std::min(0.6 * (double)free_b, 192.0 * (1ull << 30));
     int b = (int)std::max(1.0, std::floor(budget / per));

@@ -231,3 +231,46 @@ def test_solves_whose_waits_run_out_are_errors(require_gpu):
         limit(s._handle, 0)
         s.adjoint_backward_device(one.data_ptr(), grad.data_ptr())
         assert bool(torch.isfinite(grad).all()) and float(grad.abs().max()) > 0.0
+
+
+def test_resident_batch_counts_the_chief_solves(require_gpu):
+    """128 CHIEF rows of a 642-dof sphere need about as much memory as its
+    matrices; with 1.2 GiB left on the card the 64 frequencies come in
+    batches that fit 60% of it."""
+    import torch
+    from meshes import sphere_buffers
+
+    from hornlab_metal_bem.native import HipBemSession
+
+    b = sphere_buffers(subdivisions=3)
+    rng = np.random.default_rng(8)
+    F, m, N = 64, 128, 704
+    d = rng.standard_normal((3, m))
+    pts = (0.06 * rng.uniform(0.3, 1.0, m) * d / np.linalg.norm(d, axis=0)).astype(np.float32)
+    k = np.linspace(5.0, 30.0, F).astype(np.float32)
+    q = np.ones((F, b.n_triangles), np.complex64)
+    obs = np.array([[0.0], [0.0], [2.0]], np.float32)
+    with HipBemSession.create_session(b) as s:
+        def solve(n):
+            return s.assemble_solve_evaluate_standard_neumann_batch(
+                k[:n] * 54.6, k[:n], q[:n], obs, chief_points=pts, estimate_rcond=False)
+
+        alone = solve(1)[0]
+        torch.cuda.empty_cache()
+        left = int(1.2 * 2**30)
+        held = []
+        while torch.cuda.mem_get_info()[0] > left + 2**30:
+            held.append(torch.empty(min(torch.cuda.mem_get_info()[0] - left, 2**33), dtype=torch.uint8,
+                                    device="cuda:0"))
+        free = torch.cuda.mem_get_info()[0]
+        try:
+            res = solve(F)
+        finally:
+            del held
+            torch.cuda.empty_cache()
+        size = res[0].diagnostics["resident_batch"]["size"]
+        # A, its copy and L; C, Z and three FP64 vectors per row, two solve words
+        need = size * (3 * 8 * N * N + 96 * m * N)
+        print(f"[contract] {free / 2**20:.0f} MiB left, batches of {size}: {need / 2**20:.0f} MiB", flush=True)
+        assert 1 <= size < F and need <= 0.6 * free
+        assert rel_l2(res[0].pressure, alone.pressure) < 2e-5
