@@ -95,13 +95,15 @@ def open_boundary_edges(triangles_nx3: NDArray[np.int32]) -> NDArray[np.int32]:
     if tris.size == 0:
         return np.empty((0, 2), dtype=np.int32)
     edges = np.sort(np.concatenate((tris[:, [0, 1]], tris[:, [1, 2]], tris[:, [2, 0]])), axis=1)
-    # one integer per edge (lexicographic order kept): sorting rows is 10x slower
+    # one integer per edge (lexicographic order kept): sorting rows is 10x slower.
+    # Differences of 32-bit indices and their products fit 64 bits unsigned.
+    edges = edges.astype(np.int64)
     lo = int(edges.min())
-    span = int(edges.max()) - lo + 1
-    keys, counts = np.unique((edges[:, 0] - lo).astype(np.int64) * span + (edges[:, 1] - lo),
-                             return_counts=True)
+    edges = (edges - lo).astype(np.uint64)
+    span = edges.max() + np.uint64(1)
+    keys, counts = np.unique(edges[:, 0] * span + edges[:, 1], return_counts=True)
     keys = keys[counts == 1]
-    return np.ascontiguousarray(np.stack([keys // span + lo, keys % span + lo], axis=1), dtype=np.int32)
+    return np.ascontiguousarray(np.stack([keys // span, keys % span], axis=1).astype(np.int64) + lo, dtype=np.int32)
 
 
 def signed_volume_indicator(verts: NDArray[np.float64], tris: NDArray[np.int32]) -> float:

@@ -274,3 +274,15 @@ def test_open_boundary_edges_are_the_rows_used_once(offset):
     assert got.dtype == np.int32
     assert np.array_equal(got, rows[counts == 1])
     assert open_boundary_edges(np.empty((0, 3), np.int32)).shape == (0, 2)
+
+
+@pytest.mark.parametrize("far", [2**31 - 2, 2**31 - 60])
+def test_open_boundary_edges_of_indices_far_apart(far):
+    """32-bit indices of both signs: their differences and the products of
+    those need more than 32 and 63 bits."""
+    from hornlab_metal_bem.mesh import open_boundary_edges
+
+    tris = np.array([[-2**31, -2**31 + 1, far], [-2**31 + 1, 7, far], [far, far + 1, 7]], np.int32)
+    edges = np.sort(np.concatenate((tris[:, [0, 1]], tris[:, [1, 2]], tris[:, [2, 0]])), axis=1)
+    rows, counts = np.unique(edges, axis=0, return_counts=True)
+    assert np.array_equal(open_boundary_edges(tris), rows[counts == 1])
