@@ -96,14 +96,14 @@ def open_boundary_edges(triangles_nx3: NDArray[np.int32]) -> NDArray[np.int32]:
         return np.empty((0, 2), dtype=np.int32)
     edges = np.sort(np.concatenate((tris[:, [0, 1]], tris[:, [1, 2]], tris[:, [2, 0]])), axis=1)
     # one integer per edge (lexicographic order kept): sorting rows is 10x slower.
-    # Differences of 32-bit indices and their products fit 64 bits unsigned.
     edges = edges.astype(np.int64)
-    lo = int(edges.min())
-    edges = (edges - lo).astype(np.uint64)
-    span = edges.max() + np.uint64(1)
-    keys, counts = np.unique(edges[:, 0] * span + edges[:, 1], return_counts=True)
+    lo = edges.min()
+    edges = (edges - lo).view(np.uint64)  # 32-bit indices: at most 32 bits each
+    low = np.uint64(32)
+    keys, counts = np.unique(edges[:, 0] << low | edges[:, 1], return_counts=True)
     keys = keys[counts == 1]
-    return np.ascontiguousarray(np.stack([keys // span, keys % span], axis=1).astype(np.int64) + lo, dtype=np.int32)
+    pairs = np.stack([keys >> low, keys & np.uint64(2**32 - 1)], axis=1).view(np.int64) + lo
+    return np.ascontiguousarray(pairs, dtype=np.int32)
 
 
 def signed_volume_indicator(verts: NDArray[np.float64], tris: NDArray[np.int32]) -> float:

@@ -286,3 +286,6 @@ def test_open_boundary_edges_of_indices_far_apart(far):
     edges = np.sort(np.concatenate((tris[:, [0, 1]], tris[:, [1, 2]], tris[:, [2, 0]])), axis=1)
     rows, counts = np.unique(edges, axis=0, return_counts=True)
     assert np.array_equal(open_boundary_edges(tris), rows[counts == 1])
+    for dtype in (np.float64, np.uint64, np.uint8):
+        e = open_boundary_edges(np.array([[0, 1, 2], [2, 1, 3]], dtype))
+        assert e.dtype == np.int32 and e.tolist() == [[0, 1], [0, 2], [1, 3], [2, 3]]
