@@ -321,12 +321,13 @@ void build_singular_classes(int nv, int T, const float *vtx, const int32_t *tri,
         }
     };
     {
-        constexpr size_t kPart = 8192;  // classes per task
+        // classes per task: enough to pay for a thread, and few threads for
+        // any mesh (sessions may be made on several threads at once)
+        const size_t part = std::max<size_t>(8192, (static_cast<size_t>(nclasses) + 7) / 8);
         std::vector<std::future<void>> tasks;
         for (int k = 0; k < 3; ++k)
-            for (size_t c = 0; c < cls[k].size(); c += kPart)
-                tasks.push_back(std::async(kAnyLaunch, fill, k, c,
-                                           std::min(cls[k].size(), c + kPart)));
+            for (size_t c = 0; c < cls[k].size(); c += part)
+                tasks.push_back(std::async(kAnyLaunch, fill, k, c, std::min(cls[k].size(), c + part)));
         for (auto &t : tasks) t.get();
     }
 

@@ -274,3 +274,42 @@ def test_resident_batch_counts_the_chief_solves(require_gpu):
         print(f"[contract] {free / 2**20:.0f} MiB left, batches of {size}: {need / 2**20:.0f} MiB", flush=True)
         assert 1 <= size < F and need <= 0.6 * free
         assert rel_l2(res[0].pressure, alone.pressure) < 2e-5
+
+
+def test_session_plan_starts_few_threads(require_gpu):
+    """The plan of a mesh of 80000 triangles (a million singular classes) is
+    built by a bounded number of threads: a process may make many sessions at
+    once."""
+    import os
+    import threading
+
+    from meshes import mesh_buffers
+
+    from hornlab_metal_bem.native import HipBemSession
+
+    nu, nv = 400, 100
+    i, j = np.divmod(np.arange(nu * nv), nv)
+    a, c = 2 * np.pi * i / nu, 2 * np.pi * j / nv
+    V = np.stack([(0.3 + 0.1 * np.cos(c)) * np.cos(a), (0.3 + 0.1 * np.cos(c)) * np.sin(a), 0.1 * np.sin(c)], 1)
+    at = lambda di, dj: (i + di) % nu * nv + (j + dj) % nv  # noqa: E731
+    F = np.concatenate([np.stack([at(0, 0), at(1, 0), at(1, 1)], 1), np.stack([at(0, 0), at(1, 1), at(0, 1)], 1)])
+    b = mesh_buffers(V, F.astype(np.int32), np.full(len(F), 2, np.int32))
+    with HipBemSession.create_session(horn_buffers(edge_length=0.05), symmetry_plane="yz+xz"):
+        pass  # the runtime's own threads are there
+    count = lambda: len(os.listdir("/proc/self/task"))  # noqa: E731
+    before, most, done = count(), [0], threading.Event()
+
+    def watch():
+        while not done.is_set():
+            most[0] = max(most[0], count())
+
+    t = threading.Thread(target=watch)
+    t.start()
+    try:
+        with HipBemSession.create_session(b, check_open_edges=False):
+            pass
+    finally:
+        done.set()
+        t.join()
+    print(f"[contract] threads: {before} before, at most {most[0]}", flush=True)
+    assert most[0] - before <= 1 + 12  # the watcher, the plan's 1 + 10, one spare
