@@ -134,21 +134,80 @@ def test_split_and_whole_singular_rules_agree(require_gpu):
             assert rel_l2(one[0].pressure, whole[i].pressure) < 2e-5
 
 
-@pytest.mark.parametrize("n_freq", [200, 400])
-def test_whole_halved_and_quartered_runs_agree(require_gpu, n_freq):
-    """Six tile pairs per frequency: one frequency cuts the blocks in four, 200
-    in two, 400 not at all, with tables that overflow in each."""
-    b = _soup(37)
+def _check_sweep(b, plane, n_freq, tol=2e-5, **kw):
+    """A sweep in one resident batch; three of its pressures against the FP64
+    oracle: entries good to 1e-7 times the condition number with scaled rows
+    (soups 5, the fan 14, the horns up to 170)."""
     f = np.geomspace(300.0, 1500.0, n_freq)
     k = (2 * np.pi * f / 343.0).astype(np.float32)
     q = np.ones((n_freq, b.n_triangles), np.complex64)
     obs = np.array([[0.0], [0.0], [2.0]], np.float32)
-    with _session(b) as s:
-        batch = s.assemble_solve_evaluate_standard_neumann_batch(f, k, q, obs)
-        for i in (0, n_freq // 2, n_freq - 1):
-            one = s.assemble_solve_evaluate_standard_neumann_batch(f[i:i + 1], k[i:i + 1], q[i:i + 1], obs)
-            # FP32 rounding times cond (separate triangles: below 100)
-            assert rel_l2(batch[i].pressure, one[0].pressure) < 2e-5
+    with _session(b, plane) as s:
+        r = s.assemble_solve_evaluate_standard_neumann_batch(
+            f, k, q, obs, batch_frequencies=n_freq, estimate_rcond=False, **kw)
+    assert all(x.diagnostics["resident_batch"]["size"] == n_freq for x in r)
+    g = O.Geometry.from_buffers(b, plane)
+    for i in sorted({0, n_freq // 2, n_freq - 1}):
+        A, rhs, _ = O.assemble(g, float(k[i]), q[i])
+        assert rel_l2(r[i].pressure, O.solve(A, rhs)) < tol, i
+
+
+@pytest.mark.parametrize("plane", [None, "yz+xz"])
+@pytest.mark.parametrize("n_freq", [1, 200, 400])
+def test_whole_halved_and_quartered_runs(require_gpu, n_freq, plane):
+    """Tables that overflow, three tiles and so six tile pairs per frequency:
+    6 blocks are cut in four, 1200 in two, 2400 (2048 and more) not at all."""
+    _check_sweep(_soup(37), plane, n_freq)
+
+
+@pytest.mark.parametrize("n_freq", [1, 400, 700])
+def test_long_column_lists_whole_halved_and_quartered(require_gpu, n_freq):
+    """Two tiles, three tile pairs per frequency: 3, 1200 and 2100 blocks."""
+    _check_sweep(_fan(40), None, n_freq)
+
+
+@pytest.mark.parametrize("body,plane", [("soup", None), ("soup", "xz"), ("soup", "yz+xz"), ("fan", None),
+                                        ("horn", None), ("horn", "xz"), ("horn", "yz+xz")])
+def test_fp64_geometry_with_full_tables_and_long_lists(require_gpu, body, plane):
+    b = {"soup": lambda: _soup(37), "fan": lambda: _fan(40), "horn": lambda: horn_buffers(edge_length=0.03)}[body]()
+    _check_sweep(b, plane, 3, precise_geometry=True)
+
+
+@pytest.mark.parametrize("plane", [None, "xz", "yz+xz"])
+def test_group_with_full_tables_and_long_lists(require_gpu, plane):
+    """Members in one launch: overflowing tables beside a member whose tables
+    do not, and (without planes) long lists."""
+    import torch
+
+    from hornlab_metal_bem.native import GroupCase, HipBemGroup
+
+    bodies = [_soup(37), _soup(30, seed=1), horn_buffers(edge_length=0.04)] + ([_fan(40)] if plane is None else [])
+    F, dev = 2, torch.device("cuda:0")
+    k = np.array([6.0, 20.0], np.float32)
+    sessions, cases, held = [], [], []
+    try:
+        for b in bodies:
+            t = dict(k=torch.as_tensor(k, device=dev),
+                     q=torch.ones((F, b.n_triangles), dtype=torch.complex64, device=dev),
+                     obs=torch.tensor([[0.0], [0.0], [2.0]], device=dev),
+                     field=torch.zeros((F, 1), dtype=torch.complex64, device=dev),
+                     p=torch.zeros((F, b.p1_dof_count), dtype=torch.complex64, device=dev),
+                     tag=torch.zeros((F, 2), dtype=torch.complex128, device=dev))
+            held.append(t)
+            sessions.append(_session(b, plane))
+            a = {n: v.data_ptr() for n, v in t.items()}
+            cases.append(GroupCase(F, a["k"], a["k"], a["q"], 1, a["obs"], a["field"], a["tag"], a["p"]))
+        torch.cuda.synchronize()
+        with HipBemGroup(sessions) as group:
+            group.solve_device(cases, source_tags=[2], impedance_source_tag=2)
+        for b, t in zip(bodies, held):
+            for i in range(F):
+                A, rhs, _ = O.assemble(O.Geometry.from_buffers(b, plane), float(k[i]),
+                                       np.ones(b.n_triangles, np.complex64))
+                assert rel_l2(t["p"][i].cpu().numpy(), O.solve(A, rhs)) < 2e-5  # as in _check_sweep
+    finally:
+        for s in sessions:
+            s.close()
 
 
 def _field_terms(b, p, q, obs):
@@ -238,7 +297,7 @@ def test_growing_waves_stay_finite(require_gpu, plane, precise):
                              k_imag_ptr=dev["kim"].data_ptr(), p_ptr=p.data_ptr(), source_tags=[2],
                              precise_geometry=precise)
     A, rhs, _ = O.assemble(O.Geometry.from_buffers(b, plane), k, q, kim=kim)
-    assert rel_l2(p.cpu().numpy(), O.solve(A, rhs)) < 2e-5  # cond(A) ~ 30
+    assert rel_l2(p.cpu().numpy(), O.solve(A, rhs)) < 2e-5  # entries good to 1e-7, condition 110 with scaled rows
 
 
 def test_coincident_points_with_fp64_geometry(require_gpu):
@@ -255,4 +314,4 @@ def test_coincident_points_with_fp64_geometry(require_gpu):
             np.array([1000.0]), np.array([20.0], np.float32), q, np.array([[0.0], [0.0], [2.0]], np.float32),
             precise_geometry=True)[0]
     A, rhs, _ = O.assemble(O.Geometry.from_buffers(b), 20.0, q[0])
-    assert rel_l2(r.pressure, O.solve(A, rhs)) < 2e-5  # cond(A) below 100
+    assert rel_l2(r.pressure, O.solve(A, rhs)) < 2e-5  # condition 4 with scaled rows
