@@ -262,14 +262,18 @@ def test_c5_adjoint_directional_derivatives_match_gpu_forward(require_gpu):
     """~3000-dof quarter horn, 24 frequencies: the hand-written adjoint's
     derivative of the directivity/ripple loss along the gradient and along a
     random direction of the off-plane vertices against central differences
-    of the same loss through the GPU forward, Richardson-extrapolated from
-    two steps (the loss's curvature in dB is large near the directivity
-    nulls; the extrapolation removes the step^2 term).  Along the gradient
-    the derivative is |G| and steps of 4e-5 and 2e-5 m keep the curvature
-    term small; along the random direction it is ~3e-3 |G|, so the steps are
-    1.6e-4 and 8e-5 m: with 2e-5 m the loss changes by ~1e-3 of ~417, where
-    the FP32 forward's evaluation-to-evaluation noise moves the difference
-    quotient by several units."""
+    of the same loss through the GPU forward, extrapolated to step 0 in even
+    powers of the step (the loss's curvature in dB is large near the
+    directivity nulls).  The FP32 forward moves the loss (~417) by 3e-4 from
+    one step to the next whatever the step, so a difference quotient at
+    2e-5 m carries 1.6e-3 |G| of noise and two steps of 2e-5 and 4e-5 m
+    extrapolate with a deviation of 2.1e-3 |G|.  80 steps from 2e-5 to
+    5.6e-5 m, fitted to the fourth power with the weights of that noise,
+    deviate by 4e-4 |G| and leave at most 4e-4 |G| of the sixth power
+    (from the quotients up to 1.6e-4 m).
+    Along the random direction the derivative is ~3e-3 |G| and its curvature
+    small: two steps of 8e-5 and 1.6e-4 m, to the second power, deviate by
+    4e-4 |G|."""
     import torch
 
     from hornlab_metal_bem.adjoint import FieldProblem, directivity_ripple_loss, exterior_field
@@ -299,17 +303,16 @@ def test_c5_adjoint_directional_derivatives_match_gpu_forward(require_gpu):
     dirs = {"gradient": np.where(off[None], G, 0.0),
             "random": np.where(off[None], rng.standard_normal(V0.shape), 0.0)}
     scale = float(np.linalg.norm(dirs["gradient"]))  # |G| on the moved vertices
-    steps = {"gradient": (4e-5, 2e-5), "random": (1.6e-4, 8e-5)}
+    steps = {"gradient": (np.geomspace(2e-5, 5.6e-5, 80), 2), "random": (np.array([8e-5, 1.6e-4]), 1)}
     for name, d in dirs.items():
         d = d / np.linalg.norm(d)
-        fds = []
-        for eps in steps[name]:
-            Lp, _ = loss_at(V0 + eps * d)
-            Lm, _ = loss_at(V0 - eps * d)
-            fds.append((Lp - Lm) / (2 * eps))
-        fd = (4.0 * fds[1] - fds[0]) / 3.0
+        eps, degree = steps[name]
+        fds = np.array([(loss_at(V0 + e * d)[0] - loss_at(V0 - e * d)[0]) / (2 * e) for e in eps])
+        x = eps / eps.max()  # the weights: noise ~ 1 / step
+        powers = np.stack([x ** (2 * j) for j in range(degree + 1)], axis=1)
+        fd = float(np.linalg.lstsq(powers * x[:, None], fds * x, rcond=None)[0][0])
         an = float(np.sum(G * d))
-        _log(f"c5 {name}: adjoint {an:.6e} central differences {fds[0]:.6e} {fds[1]:.6e} "
+        _log(f"c5 {name}: adjoint {an:.6e} central differences {fds[0]:.6e} to {fds[-1]:.6e} "
              f"extrapolated {fd:.6e}, error / |G| {abs(fd - an) / scale:.2e}")
         assert abs(fd - an) <= 2e-3 * scale, (name, an, fds)
 
