@@ -1612,13 +1612,23 @@ void launch_assemble_regular(const DeviceGeometry &g, int n_batch, const float *
                              float *A, int64_t lda, int64_t a_stride, float *rhs,
                              int64_t rhs_stride, hipStream_t stream, bool precise) {
     if (g.n_tile_pairs == 0 || n_batch <= 0) return;
-    // Two blocks fit a CU.  A launch of a few rounds loses most of its last one,
-    // and one of less than a round leaves CUs idle: its blocks are cut in two or
-    // four (each then writes its rows to A on its own): 528 blocks (1078 dofs, one
-    // frequency) 0.505 ms whole, 0.422 in four.  The FP64-geometry variant runs
-    // whole (registers).
+    // Two blocks fit a CU, 512 the card.  Where blocks leave slots idle they are
+    // cut in two or four, each part writing its rows to A on its own; with
+    // images a block carries two or four times the work of its writes, and
+    // halves also pay while the last round of a launch weighs.  Kernel times in
+    // us whole / in two / in four, at blocks:
+    //   1 image   105: 108/73/70   180: 128/108/131   315: 151/164/175   903: 298/320/399
+    //   2 images  112: 149/83/72   171: 149/114/130   513: 266/245/265   2052: 760/778/868
+    //   4 images  112: 255/142/105 528: 510/423/418   1056: 793/742/767  2112: 1390/1383/1456
+    // The FP64-geometry variant runs whole (registers).
     const int64_t blocks = (int64_t)g.n_tile_pairs * n_batch;
-    const int parts = precise || blocks >= 2048 ? 1 : (blocks >= 1024 ? 2 : 4);
+    int parts = 1;
+    if (!precise) {
+        if (blocks <= 128 || (g.n_masks == 4 && blocks <= 512))
+            parts = 4;
+        else if (blocks <= 256 || (g.n_masks > 1 && blocks < 2048))
+            parts = 2;
+    }
     dim3 grid(g.n_tile_pairs * parts, n_batch);
     const size_t shm = 64 * (size_t)regular_wave_lds(g.run_rows, g.max_tile_dofs);
     auto go = [&](auto complex_k, auto masks) {
