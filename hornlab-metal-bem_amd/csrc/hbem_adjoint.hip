@@ -101,9 +101,10 @@ __device__ __forceinline__ AdjK adj_kernel_far(double dx, double dy, double dz, 
 
 // 1/r and the reduced phase (revolutions) of six distances given as r^2 in
 // FP64, then sin and cos: the transcendentals of six evaluations as one run at
-// raised wave priority; both zero (so G is) for r^2 <= 1e-14.  A transcendental takes both issue ports of a SIMD for
-// 8 cycles; interleaved with FP32 work it also keeps two waves from pairing
-// their operations.  kComplexK: damp = e^{-k_im r}.
+// raised wave priority; both zero (so G is) for r^2 <= 1e-14.  A transcendental
+// takes both issue ports of a SIMD for 8 cycles; interleaved with FP32 work it
+// also keeps two waves from pairing their operations.  kComplexK: damp =
+// e^{-k_im r}.
 template <bool kComplexK>
 __device__ __forceinline__ void adj_phases(const double (&r2d)[6], double krev, float kim,
                                            float (&rinv)[6], float (&sn)[6], float (&cs)[6],
@@ -409,8 +410,9 @@ __global__ __launch_bounds__(256) void k_residual_h_f64(const float *__restrict_
 // ---------------------------------------------------------------------------
 constexpr int kAdjTestsPerWave = 96;
 
-// Two waves per SIMD (at most 256 VGPRs; unbounded the kernel took 282 and
-// ran one wave per SIMD with its transcendental chains exposed).
+// Two waves per SIMD: at most 256 VGPRs, 17 of them spilled (complex k 21);
+// unbounded the kernel spills none but runs one wave per SIMD, which exposes
+// its dependency chains.
 template <bool kComplexK>
 __global__ __launch_bounds__(256, 2) void k_adjoint_regular(
     DeviceGeometry g, const float *__restrict__ k_real, const float *__restrict__ k_imag,

@@ -141,9 +141,10 @@ struct hbem_session {
     hipStream_t stream = nullptr;
     hbem::Plan plan;
     hbem::DeviceGeometry dg{};
-    DevBuf tri_f_aos, tri_i_aos, tri_t_f, tri_t_i, tri_f_soa, tri_i_soa, sg_f, sg_i, sg_rule, sg_rule_reg, gather, tile_groups, row_map, tile_touch, tile_start,
-        tile_count, tile_ndofs, tile_dofs, tile_pairs, nc_f, nc_i, nc_rule, sg_adj, vtx_d, triv_d,
-        normals_d, jac_d;
+    DevBuf tri_f_aos, tri_i_aos, tri_t_f, tri_t_i, tri_f_soa, tri_i_soa, sg_f, sg_i,
+        sg_rule, sg_rule_reg, gather, tile_groups, row_map, tile_touch, tile_start,
+        tile_count, tile_ndofs, tile_dofs, tile_pairs, nc_f, nc_i, nc_rule, sg_adj, vtx_d,
+        triv_d, normals_d, jac_d;
     // CHIEF rows and solves of the current resident batch
     DevBuf chief_C, chief_d, chief_pts, chief_z, chief_e, chief_z64, chief_r, chief_ainf;
     const float *chief_pts_d = nullptr;
@@ -185,11 +186,20 @@ struct hbem_session {
     int cu_count = 0;
 
     ~hbem_session() {
-        for (DevBuf *b : {&tri_f_aos, &tri_i_aos, &tri_t_f, &tri_t_i, &tri_f_soa, &tri_i_soa, &sg_f, &sg_i,
-                          &sg_rule, &sg_rule_reg, &gather, &tile_groups, &row_map, &tile_touch, &tile_start, &tile_count, &tile_ndofs, &tile_dofs, &tile_pairs, &nc_f, &nc_i, &nc_rule, &sg_adj, &vtx_d, &triv_d, &normals_d, &jac_d, &adj_k, &adj_kim, &adj_fk, &adj_q, &adj_beta, &adj_obs, &adj_c, &adj_ft, &adj_sig, &adj_gN, &adj_l32, &adj_e64, &adj_l64, &adj_r64, &adj_act, &chief_C, &chief_d, &chief_pts, &chief_z, &chief_e, &chief_z64, &chief_r, &chief_ainf, &A, &A_orig, &rhs, &x, &x64, &r64, &xprev, &ipiv, &info, &gl, &lu_scr_i, &lu_scr_f, &lu_pack, &amax, &lu_scale, &kv, &kh, &kn, &kf, &q, &kre,
-                          &kim, &fk, &obs, &field, &tags, &tagout, &norms, &anorm, &active,
-                          &rowsplit, &rcx, &rcy, &rc_state, &rc_est, &io_k, &io_kim, &io_fk, &io_q, &io_obs, &io_field,
-                          &io_p, &io_tag, &io_beta, &qt, &l2g, &lu_perm, &lu_pi, &lu_lf, &lu_dinv, &ts_ctx[0],
+        for (DevBuf *b : {&tri_f_aos, &tri_i_aos, &tri_t_f, &tri_t_i, &tri_f_soa, &tri_i_soa,
+                          &sg_f, &sg_i, &sg_rule, &sg_rule_reg, &gather, &tile_groups,
+                          &row_map, &tile_touch, &tile_start, &tile_count, &tile_ndofs,
+                          &tile_dofs, &tile_pairs, &nc_f, &nc_i, &nc_rule, &sg_adj, &vtx_d,
+                          &triv_d, &normals_d, &jac_d, &adj_k, &adj_kim, &adj_fk, &adj_q,
+                          &adj_beta, &adj_obs, &adj_c, &adj_ft, &adj_sig, &adj_gN, &adj_l32,
+                          &adj_e64, &adj_l64, &adj_r64, &adj_act, &chief_C, &chief_d,
+                          &chief_pts, &chief_z, &chief_e, &chief_z64, &chief_r, &chief_ainf,
+                          &A, &A_orig, &rhs, &x, &x64, &r64, &xprev, &ipiv, &info, &gl,
+                          &lu_scr_i, &lu_scr_f, &lu_pack, &amax, &lu_scale, &kv, &kh, &kn,
+                          &kf, &q, &kre, &kim, &fk, &obs, &field, &tags, &tagout, &norms,
+                          &anorm, &active, &rowsplit, &rcx, &rcy, &rc_state, &rc_est, &io_k,
+                          &io_kim, &io_fk, &io_q, &io_obs, &io_field, &io_p, &io_tag,
+                          &io_beta, &qt, &l2g, &lu_perm, &lu_pi, &lu_lf, &lu_dinv, &ts_ctx[0],
                           &ts_ctx[1], &ts_y[0], &ts_y[1], &ts_z[0], &ts_z[1]})
             b->release();
         if (lu_graph) (void)hipGraphExecDestroy(lu_graph);

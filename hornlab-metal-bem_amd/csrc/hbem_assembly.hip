@@ -167,7 +167,10 @@ __device__ __forceinline__ RuleWeights rule_weights() {
 
 // Basis sums of complex values; sum(j) is basis j's.  kShared: s + e[j] with
 // the shared sum above; else the three sums with their own weights (6 FMAs),
-// whose rounding stays below that of the smallest weight (FP64 geometry).
+// whose rounding stays below that of the smallest weight (FP64 geometry).  With
+// FP32 geometry the shared sums are no less accurate: over 17 meshes and
+// wavenumbers the off-diagonal entries' errors against 64 bits are 0 to 15%
+// smaller than with own weights.
 template <bool kShared>
 struct BasisSum {
     float s[2], e[3][2];
@@ -217,8 +220,8 @@ __device__ __forceinline__ float flip(float a, int mask, int c) {
 // wave-uniform (scalar registers).  The next test's records are fetched one
 // test ahead as one vector load spread over the lanes (lane l < 32: float
 // word l, lane 32 + l: int word l) and moved to scalar registers with
-// v_readlane, so waiting for them never waits for the LDS adds in flight
-// (scalar loads share their counter with LDS operations).
+// v_readlane, so waiting for them never waits for the LDS reads and writes of
+// a flush (scalar loads share their counter with LDS operations).
 struct TestRec {
     float xo[18];  // quadrature points as offsets from vertex 0
     float n[3];    // unit normal
@@ -723,7 +726,10 @@ __device__ __forceinline__ void regular_tile_pair(
         float sR[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
         const float rf = rev ? 1.0f : 0.0f;
         const bool src = wave_has_source || test_source;
-        // images in pairs: four at once hold 24 more registers than fit
+        // images in pairs: four at once hold 24 more registers than fit.  With
+        // 256 registers (two waves per SIMD) the FP32 kernels spill none (whole
+        // runs with four images and complex k 2, shares of a run up to 5, the
+        // multi-mesh kernel up to 10), those with FP64 geometry 18 to 76.
         constexpr int kGroup = kM < 2 ? kM : 2;
         auto images = [&](int m) {
             if (src)
@@ -876,8 +882,7 @@ __global__ __launch_bounds__(256, 2) void k_assemble_regular(
     float *__restrict__ rhs, int64_t rhs_stride) {
     regular_tile_pair<kComplexK, kM, kPrecise, kParts>(
         g, kParts ? blockIdx.x / parts : blockIdx.x, kParts ? blockIdx.x % parts : 0, parts,
-        blockIdx.y, k_real, k_imag, q, n_src,
-                                               beta, A, lda, a_stride, rhs, rhs_stride);
+        blockIdx.y, k_real, k_imag, q, n_src, beta, A, lda, a_stride, rhs, rhs_stride);
 }
 
 // The member of a multi-mesh launch that owns flattened block `blk`: jobs
@@ -900,15 +905,15 @@ __global__ __launch_bounds__(256, 2) void k_assemble_regular_multi(
     const AssemblyJob &jb = jobs[j];
     const int local = blockIdx.x - jb.block_begin_reg;
     const int ntp = jb.g.n_tile_pairs;
-    regular_tile_pair<kComplexK, kM, false, false>(jb.g, local % ntp, 0, 1, local / ntp, jb.k_real, jb.k_imag,
-                                            jb.q, jb.n_src, jb.beta, jb.A, jb.lda, jb.a_stride,
-                                            jb.rhs, jb.rhs_stride);
+    regular_tile_pair<kComplexK, kM, false, false>(
+        jb.g, local % ntp, 0, 1, local / ntp, jb.k_real, jb.k_imag, jb.q, jb.n_src, jb.beta, jb.A,
+        jb.lda, jb.a_stride, jb.rhs, jb.rhs_stride);
 }
 
 // ---------------------------------------------------------------------------
 // Singular pair classes.  One lane per class, kFB frequencies per lane; a
 // wave holds classes of one kind, so the Sauter-Schwab points are
-// wave-uniform and stream through scalar loads.  Per point and lane:
+// wave-uniform and come from LDS as broadcasts.  Per point and lane:
 // the distance vector from the class's affine maps (cancellation-free on
 // shared vertices and edges), one rsq, then per frequency sin/cos and the
 // fused 3x3 double-layer block plus 3 single-layer moments.  Sums run in
@@ -940,8 +945,9 @@ __device__ __forceinline__ void singular_block(
     const int part = kSplit > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
     // split groups start with the vertex pairs: the coincident ones carry the
     // mass terms, the largest summands of their entries, which round least
-    // when they are added last
-    const int w = kSplit > 1 ? g.sg_waves[0] + g.sg_waves[1] + g.sg_waves[2] - 1 - bx : __builtin_amdgcn_readfirstlane(bx * 4 + (threadIdx.x >> 6));
+    // when they are added last (blocks start in order, so they usually are)
+    const int w = kSplit > 1 ? g.sg_waves[0] + g.sg_waves[1] + g.sg_waves[2] - 1 - bx
+                             : __builtin_amdgcn_readfirstlane(bx * 4 + (threadIdx.x >> 6));
     const int w1 = g.sg_waves[0], w2 = w1 + g.sg_waves[1], w3 = w2 + g.sg_waves[2];
     if (w >= w3) return;
     const int kind = w < w1 ? 0 : (w < w2 ? 1 : 2);
