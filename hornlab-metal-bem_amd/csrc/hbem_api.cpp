@@ -127,6 +127,39 @@ struct Timer {
 
 int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
+// Pairs of words in pinned host memory (TrsvSync::expired of a session's two
+// contexts), cut from pages that are kept: a dense solve makes a session per
+// call, and pinning costs 20 us.  One page holds 512 pairs; pages are added
+// only while more sessions are alive and stay until the process ends.
+struct ExpiredWords {
+    std::mutex mu;
+    std::vector<uint32_t *> free;
+};
+ExpiredWords &expired_words() {
+    static ExpiredWords *words = new ExpiredWords;  // sessions may outlive statics
+    return *words;
+}
+uint32_t *take_expired_words() {
+    ExpiredWords &w = expired_words();
+    std::lock_guard<std::mutex> lock(w.mu);
+    if (w.free.empty()) {
+        constexpr size_t kBytes = 4096, kPairs = kBytes / (2 * sizeof(uint32_t));
+        void *page = nullptr;
+        w.free.reserve(w.free.capacity() + kPairs);
+        hip_check(hipHostMalloc(&page, kBytes, hipHostMallocPortable), "hipHostMalloc");
+        for (size_t i = 0; i < kPairs; ++i) w.free.push_back(static_cast<uint32_t *>(page) + 2 * i);
+    }
+    uint32_t *pair = w.free.back();
+    w.free.pop_back();
+    return pair;
+}
+void give_expired_words(uint32_t *pair) {
+    if (!pair) return;
+    ExpiredWords &w = expired_words();
+    std::lock_guard<std::mutex> lock(w.mu);
+    w.free.push_back(pair);  // within the capacity reserved for its page
+}
+
 }  // namespace
 
 namespace hbem {
@@ -177,7 +210,7 @@ struct hbem_session {
     DevBuf lu_perm, lu_pi, lu_lf, lu_dinv, ts_ctx[2], ts_y[2], ts_z[2];
     hbem::TrsvSync trsv[2] = {};
     bool trsv_on = false;
-    uint32_t *trsv_expired = nullptr;  // [2], pinned
+    uint32_t *trsv_expired = nullptr;  // [2], from take_expired_words
     uint32_t trsv_polls = hbem::kTrsvPolls;
     double setup_seconds = 0.0;
     int64_t near_pairs = 0;
@@ -203,7 +236,7 @@ struct hbem_session {
                           &ts_ctx[1], &ts_y[0], &ts_y[1], &ts_z[0], &ts_z[1]})
             b->release();
         if (lu_graph) (void)hipGraphExecDestroy(lu_graph);
-        if (trsv_expired) (void)hipHostFree(trsv_expired);
+        give_expired_words(trsv_expired);
         if (aux_stream) (void)hipStreamDestroy(aux_stream);
         if (ev_lu) (void)hipEventDestroy(ev_lu);
         if (stream) (void)hipStreamDestroy(stream);
@@ -312,11 +345,7 @@ hbem::TrsvSync trsv_sync(hbem_session *s, int which, int V, int N, hipStream_t s
     c.reserve(sizeof(uint32_t) * 4);
     y.reserve(sizeof(uint64_t) * words);
     z.reserve(sizeof(uint64_t) * words);
-    if (!s->trsv_expired) {
-        void *host = nullptr;
-        hip_check(hipHostMalloc(&host, 2 * sizeof(uint32_t), hipHostMallocDefault), "hipHostMalloc");
-        s->trsv_expired = static_cast<uint32_t *>(host);
-    }
+    if (!s->trsv_expired) s->trsv_expired = take_expired_words();
     s->trsv_expired[which] = 0;
     const hbem::TrsvSync sync{c.as<uint32_t>(), y.as<uint64_t>(), z.as<uint64_t>(),
                               s->trsv_expired + which, s->trsv_polls};
