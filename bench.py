@@ -32,13 +32,18 @@ ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT / "hornlab-metal-bem_amd"))
 
 PEAK_FP32_TFLOPS = 157.3  # MI355X FP32 vector, published
-FLOPS_PER_EVAL = 80  # G + dG/dn evaluation incl. block accumulation (fixed count)
-TRANS_PER_EVAL = 4  # sqrt/rcp, sin, cos, (exp) per evaluation (fixed count)
+# FP32 flops and transcendentals k_assemble_regular executes per evaluation of G and dG/dn incl.
+# its block accumulation, by number of images: one computed evaluation serves both directions of
+# a pair.  rocprofv3 SQ_INSTS_VALU_{ADD,MUL,FMA,TRANS}_F32, idle lanes included
+# (profiles/kernels_c2_quarter_horn_bench.md).  An evaluation by itself takes 80 flops and 4
+# transcendentals.
+FLOPS_PER_EVAL = {4: 28.2, 1: 33.3}
+TRANS_PER_EVAL = 1.6
 REFERENCE_FREQ_PER_S = 20.0  # reference README: 40 freqs in ~2 s on Apple M-series
 # HBM bytes per k_assemble_regular dispatch of one sweep of the default mesh
 # of each workload: rocprofv3 FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000 (factors
 # from a 512 MiB copy kernel), profiles/pmc_traffic_c2_regular_assembly.md
-REGULAR_TRAFFIC_BYTES: dict[str, float] = {"c2": 3.208e9}
+REGULAR_TRAFFIC_BYTES: dict[str, float] = {"c2": 3.281e9}
 
 
 WORKLOADS = {
@@ -513,7 +518,7 @@ def main() -> int:
     reg_launch_s = reg_ms * 1e-3 / launches_per_step
     n_img = 4 if sym == "yz+xz" else (1 if sym is None else 2)
     evals_per_step = float(T) ** 2 * 36 * n_img * F
-    achieved = evals_per_step / launches_per_step * FLOPS_PER_EVAL / reg_launch_s / 1e12
+    achieved = evals_per_step / launches_per_step * FLOPS_PER_EVAL[n_img] / reg_launch_s / 1e12
 
     # transcendental side of the assembly roofline: rsq + sin + cos per
     # computed pair-point evaluation, each serving both directed blocks
@@ -633,7 +638,7 @@ def main() -> int:
             "frac": round(achieved / PEAK_FP32_TFLOPS, 4),
             "traffic": REGULAR_TRAFFIC_BYTES.get(args.workload) if args.dofs is None else None,
             "algorithmic": f"T^2*36*(1+I)*F = {evals_per_step:.4g} G/dG evaluations per step x "
-            f"{FLOPS_PER_EVAL} FP32 flops (+{TRANS_PER_EVAL} transcendentals) each",
+            f"{FLOPS_PER_EVAL[n_img]} FP32 flops (+{TRANS_PER_EVAL} transcendentals) executed each",
             "launch_ms": round(reg_launch_s * 1e3, 4),
         },
         "roofline_transcendental": trans,

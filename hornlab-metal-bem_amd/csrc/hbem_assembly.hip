@@ -1389,8 +1389,8 @@ struct FieldPoint {
     float off_n, pad;
 };
 
-// Bound by the VALU: per evaluation 15 FP64 operations and conversions, 14 FP32
-// operations and 3 transcendentals.  Distance and phase are formed in FP64: a
+// Bound by the VALU: 42 operations per evaluation with four images (18 FP32, 3
+// transcendentals, the rest FP64 and conversions), 49 without.  Distance and phase are formed in FP64: a
 // point 2 m away keeps the phase accuracy of the surface, and one a tenth of an
 // element from it does not lose its distance to the cancellation of vertex and
 // offset (FP32 differences, 5% faster: errors 10 to 50 times as large at 0.2 to
