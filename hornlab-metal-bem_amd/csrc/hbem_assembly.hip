@@ -1621,8 +1621,8 @@ void launch_assemble_regular(const DeviceGeometry &g, int n_batch, const float *
     // Two blocks fit a CU, 512 the card.  Where blocks leave slots idle they are
     // cut in two or four, each part writing its rows to A on its own; with
     // images a block carries two or four times the work of its writes, and
-    // halves also pay while the last round of a launch weighs.  Kernel times in
-    // us whole / in two / in four, at blocks:
+    // halves also pay while the few blocks left at a launch's end weigh.  Kernel
+    // times in us whole / in two / in four, at blocks:
     //   1 image   105: 108/73/70   180: 128/108/131   315: 151/164/175   903: 298/320/399
     //   2 images  112: 149/83/72   171: 149/114/130   513: 266/245/265   2052: 760/778/868
     //   4 images  112: 255/142/105 528: 510/423/418   1056: 793/742/767  2112: 1390/1383/1456
